@@ -225,6 +225,38 @@ def test_getrf_f32_leaf_geometry_does_not_change_the_factors():
     assert torch.equal(default.a[:, :n], wide.a[:, :n])
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [63, 65, 256, 257, 512, 513, 768, 769, 1024, 1025])
+def test_getrf_lone_leaves_match_exchanging_leaves(dtype, n):
+    """Leaves of at most 768 (FP64) or 1024 (FP32) rows run in one workgroup
+    that exchanges nothing.  A cap on the workgroups keeps the exchanging
+    leaves: same factors and pivots, bit for bit, and LAPACK's info for an
+    exactly zero column."""
+    from updes_amd import engine as E
+    L = _lib()
+    a = _random_well(n, 3 * n)
+    zero = n // 2
+    for col in (None, zero):
+        if col is not None:
+            a[:, col] = 0.0
+        m = torch.zeros((n, E._ld(n)), dtype=dtype)
+        m[:, :n] = torch.as_tensor(a).to(dtype)
+        lone = E.LU(m.cuda(), n)
+        L.check(L.lib().rbfx_set_panel_groups(4))
+        try:
+            shared = E.LU(m.cuda(), n)
+            torch.cuda.synchronize()
+        finally:
+            L.check(L.lib().rbfx_set_panel_groups(0))
+        assert torch.equal(lone.ipiv, shared.ipiv)
+        assert torch.equal(lone.a[:, :n], shared.a[:, :n])
+        assert lone.singular == shared.singular == (0 if col is None else col + 1)
+    if dtype == torch.float64:
+        a = _random_well(n, 3 * n)
+        m[:, :n] = torch.as_tensor(a)
+        assert np.array_equal(E.LU(m.cuda(), n).ipiv.cpu().numpy(), sla.lu_factor(a)[1])
+
+
 def test_getrf_matches_lapack_pivots():
     """Same pivot sequence as LAPACK getrf on a matrix without ties."""
     from updes_amd import engine as E

@@ -451,15 +451,24 @@ struct PanelArgs {
   int64_t left, right;  // columns of the enclosing outer panel left / right of the leaf
   int64_t* ipiv;  // (w) absolute pivot rows
   double* cand;   // [2][G][kRecWords] tagged (|value|, row) records (first two words used)
-  T* cand_row;    // [2][G][w]
+  unsigned long long* cand_row;  // [2][G][kRowStride<T>] tagged words of the candidate rows
   unsigned seq_base;  // step count before this launch
   int* status;
   int32_t* info;
   uint64_t wait_ticks;  // real-time bound of each wait (wall_clock64 ticks)
 };
 
-constexpr int kPanelThreads = 256;
+constexpr int kPanelThreads = 256;     // leaf workgroups that run beside a trailing update
 constexpr int kPanelWMax = 64;
+// A published row entry carries its own tag: each 64-bit word holds 32 bits
+// of the value and the 32-bit tag of its column, so a reader that finds the
+// tag has the value, and the writer need not wait between the row and the
+// record that announces it.
+template <typename T>
+constexpr int kRowWords = sizeof(T) / 4;
+// a published row: kPanelWMax entries and the reciprocal of the first
+template <typename T>
+constexpr int kRowStride = (kPanelWMax + 2) * kRowWords<T>;
 // Narrow leaves for the panels that run beside a long trailing update: a
 // 16-wide FP64 leaf (67 VGPRs) shares a CU with two trailing-update
 // workgroups (2 x 216 VGPRs per SIMD), where a 64-wide one (164) displaces
@@ -477,14 +486,6 @@ static std::atomic<int64_t> g_narrow_leaf_rows{0};
 // polls every record, and records sharing a line would serialise the polls.
 constexpr int kRecWords = 16;
 
-// (value, index) maximum with the smaller index winning ties.
-__device__ inline void argmax_merge(double& v, int64_t& i, double ov, int64_t oi) {
-  if (ov > v || (ov == v && oi < i)) {
-    v = ov;
-    i = oi;
-  }
-}
-
 // Pivot keys.  A candidate (|value|, row) is compared as one 64-bit key:
 // the bits of |value| with the low kKeyLow bits replaced by the position of
 // the row, inverted so that a lower position wins a tie of the truncated
@@ -495,6 +496,7 @@ __device__ inline void argmax_merge(double& v, int64_t& i, double ov, int64_t oi
 constexpr int kKeyLow = 20;
 constexpr unsigned long long kKeyValMask = ~((1ull << kKeyLow) - 1);
 constexpr int kKeyMaxGroups = 512, kKeyMaxRows = 2048;
+constexpr unsigned long long kKeyBad = ~0ull;  // not a key (a NaN value): the exchange failed
 
 __device__ inline unsigned long long pivot_key(double absval, int q, int local) {
   if (!(absval >= 0.0)) return 0ull;
@@ -502,46 +504,69 @@ __device__ inline unsigned long long pivot_key(double absval, int q, int local) 
          ((unsigned long long)(kKeyMaxGroups - 1 - q) << 11) | (unsigned long long)(kKeyMaxRows - 1 - local);
 }
 
-// Maximum of a 64-bit key over the wave with DPP row shifts and broadcasts
-// (no LDS traffic): an inclusive max-scan inside each row of 16 lanes, then
-// row 15 -> rows 1, 3 and lane 31 -> rows 2, 3, so lane 63 holds the result.
+// Maximum of an unsigned value over lanes 0 .. 16 STEP_ROWS of the wave with
+// DPP row shifts and broadcasts (no LDS traffic): an inclusive max-scan
+// inside each row of 16 lanes, then row 15 -> rows 1, 3 and lane 31 -> rows
+// 2, 3, so lane 63 (lane 15 of a single row) holds the result.
 template <int CTRL, int ROWMASK>
-__device__ inline unsigned long long dpp_u64(unsigned long long v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, ROWMASK, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), CTRL, ROWMASK, 0xf, false);
-  return ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo;
+__device__ inline unsigned dpp_max(unsigned v) {
+  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWMASK, 0xf, false);
+  return v > o ? v : o;
+}
+template <int LANES>
+__device__ inline unsigned wave_max_u32(unsigned v) {
+  static_assert(LANES == 16 || LANES == 64, "one row or the whole wave");
+  v = dpp_max<0x111, 0xf>(v);  // row_shr:1
+  v = dpp_max<0x112, 0xf>(v);  // row_shr:2
+  v = dpp_max<0x114, 0xf>(v);  // row_shr:4
+  v = dpp_max<0x118, 0xf>(v);  // row_shr:8
+  if constexpr (LANES == 64) {
+    v = dpp_max<0x142, 0xa>(v);  // row_bcast:15
+    v = dpp_max<0x143, 0xc>(v);  // row_bcast:31
+  }
+  return (unsigned)__builtin_amdgcn_readlane((int)v, LANES - 1);
 }
 __device__ inline unsigned long long umax64(unsigned long long a, unsigned long long b) { return a > b ? a : b; }
+// Maximum of a 64-bit key: the high words first (one 32-bit step per DPP
+// move), then the low words of the lanes that hold that maximum, usually one.
+template <int LANES = 64>
 __device__ inline unsigned long long wave_max_key(unsigned long long v) {
-  v = umax64(v, dpp_u64<0x111, 0xf>(v));  // row_shr:1
-  v = umax64(v, dpp_u64<0x112, 0xf>(v));  // row_shr:2
-  v = umax64(v, dpp_u64<0x114, 0xf>(v));  // row_shr:4
-  v = umax64(v, dpp_u64<0x118, 0xf>(v));  // row_shr:8
-  v = umax64(v, dpp_u64<0x142, 0xa>(v));  // row_bcast:15
-  v = umax64(v, dpp_u64<0x143, 0xc>(v));  // row_bcast:31
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, 63);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), 63);
-  return ((unsigned long long)hi << 32) | lo;
+  const unsigned hi = (unsigned)(v >> 32), lo = (unsigned)v;
+  const unsigned mh = wave_max_u32<LANES>(hi);
+  const unsigned long long top = __ballot(hi == mh && (LANES == 64 || (threadIdx.x & 63) < LANES));
+  unsigned ml;
+  if ((top & (top - 1)) == 0)
+    ml = (unsigned)__builtin_amdgcn_readlane((int)lo, __ffsll((long long)top) - 1);
+  else
+    ml = wave_max_u32<LANES>(hi == mh ? lo : 0u);
+  return ((unsigned long long)mh << 32) | ml;
 }
 
 // Block-wide key maximum; one barrier.  s has one slot per wave and is
 // reused by a later call only after at least one more barrier.
+template <int NT>
 __device__ inline unsigned long long block_max_key(unsigned long long key, unsigned long long* s) {
+  constexpr int NW = NT / 64;
   const unsigned long long wm = wave_max_key(key);
-  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = wm;
+  const int lane = threadIdx.x & 63;
+  if (lane == 0) s[threadIdx.x >> 6] = wm;
   __syncthreads();
-  unsigned long long b = s[0];
+  if constexpr (NW <= 4) {
+    unsigned long long b = s[0];
 #pragma unroll
-  for (int q = 1; q < kPanelThreads / 64; ++q) b = umax64(b, s[q]);
-  return b;
+    for (int q = 1; q < NW; ++q) b = umax64(b, s[q]);
+    return b;
+  } else {
+    static_assert(NW <= 16, "one key per lane of a row");
+    return wave_max_key<16>(lane < NW ? s[lane] : 0ull);
+  }
 }
 
-// Position bookkeeping of the panel's row interchanges, replayed from the
-// winners (every workgroup knows them) by one wave.  Only moved rows are
-// listed: pos(p) = p unless p is in the list.
+// The rows that a leaf moves and their final positions (a row that is not
+// listed stays where it is).
 struct MoveList {
-  int64_t phys[2 * kPanelWMax];
-  int64_t pos[2 * kPanelWMax];
+  int phys[2 * kPanelWMax];
+  int pos[2 * kPanelWMax];
   int cnt;
 };
 
@@ -552,61 +577,113 @@ __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ inline int ml_find(const int64_t* keys, int cnt, int64_t key) {
-  const int lane = threadIdx.x & 63;
-  for (int base = 0; base < cnt; base += 64) {
-    const int q = base + lane;
-    const unsigned long long bal = __ballot(q < cnt && keys[q] == key);
-    if (bal) return base + __ffsll((long long)bal) - 1;
-  }
-  return -1;
-}
-
 // Staging of the interchanges applied to the panel's other columns.
 constexpr int kSwapStage = 2048;
 
+// The W words of row q's candidate (tagged with tag) to lane c < n: entry c.
+template <typename T>
+__device__ inline void st_row_entry(unsigned long long* row, int c, T v, unsigned tag) {
+  const unsigned long long t = (unsigned long long)tag << 32;
+  if constexpr (sizeof(T) == 8) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    st_coh(row + 2 * c, (b & 0xFFFFFFFFull) | t);
+    st_coh(row + 2 * c + 1, (b >> 32) | t);
+  } else {
+    st_coh(row + c, (unsigned long long)__float_as_uint(v) | t);
+  }
+}
+template <typename T>
+__device__ inline bool ld_row_entry(const unsigned long long* row, int c, unsigned tag, T& v) {
+  if constexpr (sizeof(T) == 8) {
+    const unsigned long long lo = ld_coh(row + 2 * c), hi = ld_coh(row + 2 * c + 1);
+    v = __longlong_as_double((long long)((hi << 32) | (lo & 0xFFFFFFFFull)));
+    return (unsigned)(lo >> 32) == tag && (unsigned)(hi >> 32) == tag;
+  } else {
+    const unsigned long long x = ld_coh(row + c);
+    v = __uint_as_float((unsigned)x);
+    return (unsigned)(x >> 32) == tag;
+  }
+}
+
 // One leaf of the panel: columns [0, w) (w <= kPanelWMax) of rows [0, m) at
-// a.A, factored by G workgroups of kPanelThreads threads.  Thread t of
-// workgroup g holds rows g*R + t + q*kPanelThreads (q < ROWS) in registers.
-// The column loop runs over all kPanelWMax columns and rotates every row's
-// registers left by one after each column, so the current column is always
-// register 0 (no run-time register indexing) and after the loop the rows
-// are back in column order.  Columns >= w are zero and only rotated.
-template <typename T, int ROWS, int W>
-__global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelArgs<T> a) {
-  static_assert(W <= kPanelWMax, "leaf wider than the candidate rows");
-  __shared__ T urow[2 * W];  // winner row of the current column; zeros from w on
-  __shared__ unsigned long long s_k1[kPanelThreads / 64], s_k2[kPanelThreads / 64];
-  __shared__ int64_t s_win[W];
+// a.A, factored by G workgroups of NT threads.  Thread t of workgroup g
+// holds rows g*R + t + q*NT (q < ROWS) in registers.  The column loop runs
+// over all kPanelWMax columns and rotates every row's registers left by one
+// after each column, so the current column is always register 0 (no
+// run-time register indexing) and after the loop the rows are back in
+// column order.  Columns >= w are zero and only rotated.
+//
+// What bounds it is each column's chain of dependent steps, not its work:
+// the workgroup's argmax, the staging of the best row, with G > 1 two trips
+// of the exchange through the memory side of the chip (records, then the
+// winner's row; a publish-to-poll trip is ~1.2 us), and the elimination.  So
+// the row words carry their own tags (the row is not waited for before its
+// record), the owner sends the reciprocal pivot along, one wave does the
+// polling, the reduction takes 32-bit DPP steps, and the interchanges are
+// replayed in registers.  One 64-wide leaf, averaged over the leaves of an
+// LU, FP64 / FP32: 248 / 217 us at n = 10,000 (375 / 349 us with the row
+// stored and waited for first, every thread polling, 64-bit DPP steps and
+// the replay in LDS); FP32 at n = 40,000, beside the trailing update: 431 us
+// (643 us).
+template <typename T, int ROWS, int W, int NT>
+__global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {
+  static_assert(W <= kPanelWMax && W <= 64, "leaf wider than the candidate rows");
+  // [0] this workgroup's candidate row of the current column, [1] the
+  // winner's row: entry c belongs to column j + c, zeros from column w on.
+  // The odd offset puts entry 1, the first one the elimination reads, on a
+  // 16-byte boundary.
+  constexpr int kOff = 16 / (int)sizeof(T) - 1;
+  constexpr int NW = NT / 64;
+  constexpr int kChunk = 8;
+  constexpr int kRowLds = (kOff + W + 1 + 3) / 4 * 4;  // entry W: 1 / pivot
+  __shared__ __align__(16) T s_row[2][kRowLds];
+  __shared__ unsigned long long s_k1[NW], s_k2;
+  __shared__ int s_win[W];
   __shared__ int s_zero[W];
-  __shared__ int s_bad;
+  __shared__ int s_pos[W];
   __shared__ MoveList ml;
   __shared__ T stage[kSwapStage];
 
   const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x;
+  const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int w = a.w;
   const int64_t rb = (int64_t)g * a.R;
   const int64_t re = rb + a.R < a.m ? rb + a.R : a.m;
   const int nr = re > rb ? (int)(re - rb) : 0;
 
   T P[ROWS][W];
-  bool act[ROWS];
+  // the column a row was chosen for, W while it is active, W + 1: no row
+  int won[ROWS];
+  // Rows are 512 bytes or less at a stride of lda, so a load of one entry
+  // per lane touches 64 cache lines; 16-byte loads halve (FP64) or quarter
+  // (FP32) the line visits.
+  constexpr int E = 16 / (int)sizeof(T);
+  typedef T vec_t __attribute__((ext_vector_type(E)));
+  const bool wide = w == W && a.lda % E == 0 && (reinterpret_cast<uintptr_t>(a.A) & 15) == 0;
 #pragma unroll
   for (int q = 0; q < ROWS; ++q) {
-    const int local = tid + q * kPanelThreads;
-    act[q] = local < nr;
+    const int local = tid + q * NT;
+    won[q] = local < nr ? W : W + 1;
     const T* src = a.A + (rb + local) * a.lda;
+    if (wide && local < nr) {
 #pragma unroll
-    for (int c = 0; c < W; ++c) P[q][c] = (act[q] && c < w) ? src[c] : T(0);
+      for (int c = 0; c < W; c += E) {
+        const vec_t x = *reinterpret_cast<const vec_t*>(src + c);
+#pragma unroll
+        for (int e = 0; e < E; ++e) P[q][c + e] = x[e];
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < W; ++c) P[q][c] = (local < nr && c < w) ? src[c] : T(0);
+    }
   }
-  for (int c = tid; c < 2 * W; c += kPanelThreads) urow[c] = T(0);
 
   // key of this thread's best active row in register 0 (the current column)
   auto thread_key = [&]() -> unsigned long long {
     unsigned long long k = 0;
 #pragma unroll
     for (int q = 0; q < ROWS; ++q)
-      if (act[q]) k = umax64(k, pivot_key((double)fabs(P[q][0]), 0, tid + q * kPanelThreads));
+      if (won[q] == W) k = umax64(k, pivot_key((double)fabs(P[q][0]), 0, tid + q * NT));
     return k;
   };
   unsigned long long* recs = reinterpret_cast<unsigned long long*>(a.cand);
@@ -622,78 +699,122 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelArgs<T> a) {
       P[q][W - 1] = t0;
     }
   };
+  // bounded polling of one value by this lane; false when the factorisation
+  // has failed elsewhere or the wait expired
+  auto poll = [&](auto&& ready) -> bool {
+    if (ready()) return true;
+    uint32_t spins = 0;
+    WaitClock clk(a.wait_ticks);
+    for (;;) {
+      __builtin_amdgcn_s_sleep(1);
+      ++spins;
+      if (ready()) return true;
+      if ((spins & 255u) == 0 && __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
+        return false;
+      if (clk.expired()) {
+        __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+      }
+    }
+  };
+  // the rows have arrived: without this the loop would wait for every memory
+  // operation in flight at its top, the published row's stores included
+  __builtin_amdgcn_s_waitcnt(0xF70);
   for (int j = 0; j < w; ++j) {
+    // best active row of this workgroup for column j
+    const unsigned long long k1 = block_max_key<NT>(thread_key(), s_k1);
     const int par = j & 1;
-    const unsigned long long tag = (unsigned long long)((a.seq_base + (unsigned)(j + 1)) & 0xFFFFu);
-    // 1. best active row of this workgroup for column j
-    if (tid == 0) s_bad = 0;
-    const unsigned long long k1 = block_max_key(thread_key(), s_k1);
+    const unsigned seq = a.seq_base + (unsigned)(j + 1);
+    const unsigned long long tag = seq & 0xFFFFu;
     const int blocal = kKeyMaxRows - 1 - (int)(k1 & (kKeyMaxRows - 1));
-    // 2. publish it.  The owner of that row stores the row (absolute column
-    //    order), waits until the stores have completed, then stores the
-    //    tagged record
+    const int ow = k1 != 0 ? __builtin_amdgcn_readfirstlane((blocal % NT) >> 6) : 0;
+    // 1. the wave that holds the best row stages it in LDS with its
+    //    reciprocal pivot (the owning lane writes, then lane c reads entry c;
+    //    a wave's LDS accesses stay in order) and, with other workgroups to
+    //    tell, publishes it: the row in tagged words and, without waiting for
+    //    those stores, the record
     //      w0 = bits of |value| with the 16 low mantissa bits set to the tag,
     //      w1 = tag << 48 | row.
     //    A reader takes a record only when both words carry the tag of
-    //    column j, so the record needs no separate flag and its two stores
-    //    no order.  With no candidate, thread 0 publishes value -1.
-    const bool owner = k1 != 0 && (blocal % kPanelThreads) == tid;
-    if (owner) {
-      T* dst = a.cand_row + ((int64_t)par * G + g) * w;
-      const int qo = blocal / kPanelThreads;
-#pragma unroll
-      for (int q = 0; q < ROWS; ++q)
-        if (q == qo) {
-#pragma unroll
-          for (int c = 0; c < W; ++c)
-            if (j + c < w) st_coh(dst + j + c, P[q][c]);
-        }
-      __builtin_amdgcn_s_waitcnt(0);
-    }
-    if (owner || (k1 == 0 && tid == 0)) {
-      const double bv = k1 ? __longlong_as_double((long long)(k1 & kKeyValMask)) : -1.0;
-      const int64_t bi = k1 ? rb + blocal : INT64_MAX;
-      unsigned long long* rec = recs + kRecWords * ((int64_t)par * G + g);
-      st_coh(rec, (unsigned long long)(__double_as_longlong(bv) & ~0xFFFFll) | tag);
-      st_coh(rec + 1, (tag << 48) | ((unsigned long long)bi & 0xFFFFFFFFFFFFull));
-    }
-    // 3.-4. every workgroup's record of column j (one thread each) and the
-    //    winner across workgroups
-    unsigned long long k2 = 0;
-    for (int q = tid; q < G; q += kPanelThreads) {
-      const unsigned long long* o = recs + kRecWords * ((int64_t)par * G + q);
-      unsigned long long w0 = ld_coh(o), w1 = ld_coh(o + 1);
-      uint32_t spins = 0;
-      WaitClock clk(a.wait_ticks);
-      while ((w0 & 0xFFFFull) != tag || (w1 >> 48) != tag) {
-        __builtin_amdgcn_s_sleep(1);
-        ++spins;
-        if ((spins & 255u) == 0 &&
-            __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-          s_bad = 1;
-          break;
-        }
-        if (clk.expired()) {
-          __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          s_bad = 1;
-          break;
-        }
-        w0 = ld_coh(o);
-        w1 = ld_coh(o + 1);
+    //    column j, and a row entry only when its words do, so no store
+    //    waits for another.  With no candidate, value -1 is published.
+    if (k1 != 0 && wid == ow) {
+      const int qo = blocal / NT;
+      unsigned long long* row = a.cand_row + ((int64_t)par * G + g) * kRowStride<T>;
+      if (G > 1 && lane == 0) {
+        const double bv = __longlong_as_double((long long)(k1 & kKeyValMask));
+        unsigned long long* rec = recs + kRecWords * ((int64_t)par * G + g);
+        st_coh(rec, (unsigned long long)(__double_as_longlong(bv) & ~0xFFFFll) | tag);
+        st_coh(rec + 1, (tag << 48) | ((unsigned long long)(rb + blocal) & 0xFFFFFFFFFFFFull));
       }
-      const double ov = __longlong_as_double((long long)(w0 & ~0xFFFFull));
-      if (ov >= 0.0)
-        k2 = umax64(k2, pivot_key(ov, q, (int)((int64_t)(w1 & 0xFFFFFFFFFFFFull) - (int64_t)q * a.R)));
+      T piv = T(0);
+      if (lane == (blocal & 63)) {
+#pragma unroll
+        for (int q = 0; q < ROWS; ++q)
+          if (q == qo) {
+            piv = P[q][0];
+#pragma unroll
+            for (int c = 0; c < W; ++c) s_row[0][kOff + c] = P[q][c];
+          }
+      }
+      wave_sync();
+      if (lane < W && j + lane >= w) s_row[0][kOff + lane] = T(0);
+      if (G > 1) {
+        wave_sync();
+        if (j + lane < w) st_row_entry(row, lane, s_row[0][kOff + lane], seq);
+      }
+      if (lane == (blocal & 63)) {
+        const T rp = piv != T(0) ? T(1) / piv : T(0);
+        if (G > 1)
+          st_row_entry(row, kPanelWMax, rp, seq);
+        else
+          s_row[0][kOff + W] = rp;
+      }
+    } else if (G > 1 && k1 == 0 && tid == 0) {
+      unsigned long long* rec = recs + kRecWords * ((int64_t)par * G + g);
+      st_coh(rec, (unsigned long long)(__double_as_longlong(-1.0) & ~0xFFFFll) | tag);
+      st_coh(rec + 1, (tag << 48) | 0xFFFFFFFFFFFFull);
     }
-    k2 = block_max_key(k2, s_k2);
-    if (s_bad) return;
-    const int wq = kKeyMaxGroups - 1 - (int)((k2 >> 11) & (kKeyMaxGroups - 1));
-    const int64_t wi = (int64_t)wq * a.R + (kKeyMaxRows - 1 - (int)(k2 & (kKeyMaxRows - 1)));
-    if (k2 != 0 && (wq >= G || wi >= a.m)) {
-      // a key that names no row cannot come from the records: stop
-      if (tid == 0) __hip_atomic_store(a.status, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return;
+    // 2. one wave polls every workgroup's record of column j (a lane each),
+    //    picks the winner (the same in every workgroup) and fetches its row;
+    //    not the publishing wave, whose loads would wait for its stores
+    if (G > 1 && wid == (ow + 1) % NW) {
+      unsigned long long k2 = 0;
+      bool ok = true;
+      for (int q = lane; q < G; q += 64) {
+        const unsigned long long* o = recs + kRecWords * ((int64_t)par * G + q);
+        unsigned long long w0 = 0, w1 = 0;
+        ok = ok && poll([&]() {
+          w0 = ld_coh(o);
+          w1 = ld_coh(o + 1);
+          return (w0 & 0xFFFFull) == tag && (w1 >> 48) == tag;
+        });
+        const double ov = __longlong_as_double((long long)(w0 & ~0xFFFFull));
+        if (ok && ov >= 0.0)
+          k2 = umax64(k2, pivot_key(ov, q, (int)((int64_t)(w1 & 0xFFFFFFFFFFFFull) - (int64_t)q * a.R)));
+      }
+      k2 = wave_max_key(k2);
+      const int wq = kKeyMaxGroups - 1 - (int)((k2 >> 11) & (kKeyMaxGroups - 1));
+      if (k2 != 0 && wq < G) {
+        T v = T(0), rp = T(0);
+        if (j + lane < w) {
+          const unsigned long long* row = a.cand_row + ((int64_t)par * G + wq) * kRowStride<T>;
+          ok = ok && poll([&]() {
+            const bool r1 = lane != 0 || ld_row_entry(row, kPanelWMax, seq, rp);
+            return ld_row_entry(row, lane, seq, v) && r1;
+          });
+        }
+        if (lane < W) s_row[1][kOff + lane] = v;
+        if (lane == 0) s_row[1][kOff + W] = rp;
+      }
+      const bool bad = __ballot(!ok) != 0;
+      if (lane == 0) s_k2 = bad ? kKeyBad : k2;
     }
+    __syncthreads();
+    const T* urow = &s_row[0][0] + (G > 1 ? kRowLds : 0) + kOff;
+    const unsigned long long k2 = G > 1 ? s_k2 : k1;
+    const T piv = urow[0], rpiv = urow[W];
+    if (k2 == kKeyBad) return;
     if (k2 == 0) {
       // no finite candidate anywhere (NaN column): every workgroup sees the
       // same key, so all of them leave here together
@@ -703,88 +824,110 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelArgs<T> a) {
       }
       return;
     }
-    if (tid < w) urow[tid] = ld_coh(a.cand_row + ((int64_t)par * G + wq) * w + tid);
-    if (tid == 0) s_win[j] = wi;
-#pragma unroll
-    for (int q = 0; q < ROWS; ++q)
-      if (rb + tid + q * kPanelThreads == wi) act[q] = false;
-    __syncthreads();
-    // 5. eliminate column j from the active rows: register c holds column
+    const int wq = G > 1 ? kKeyMaxGroups - 1 - (int)((k2 >> 11) & (kKeyMaxGroups - 1)) : 0;
+    const int wi = wq * (int)a.R + (kKeyMaxRows - 1 - (int)(k2 & (kKeyMaxRows - 1)));
+    if (wq >= G || wi >= (int)a.m) {
+      // a key that names no row cannot come from the records: stop
+      if (tid == 0) __hip_atomic_store(a.status, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+    if (tid == 0) {
+      s_win[j] = wi;
+      s_zero[j] = piv == T(0);
+    }
+    // 3. eliminate column j from the active rows: register c holds column
     //    j + c (urow beyond w is zero, which also leaves the finished
-    //    columns rotated to the top untouched)
-    const T piv = urow[j];
-    const T rpiv = piv != T(0) ? T(1) / piv : T(0);
-    if (tid == 0) s_zero[j] = piv == T(0);
-    // Branch-free: an inactive row takes multiplier 0 (a divergent branch
-    // here makes the compiler keep a second copy of the row registers).
-    // Eliminated and rotated in one pass: register c takes column j+1+c,
-    // the top register the multiplier of column j.
+    //    columns rotated to the top untouched).  Branch-free: an inactive
+    //    row takes multiplier 0 (a divergent branch here makes the compiler
+    //    keep a second copy of the row registers).  Eliminated and rotated
+    //    in one pass: register c takes column j+1+c, the top register the
+    //    multiplier of column j.
+    T l[ROWS], top[ROWS];
 #pragma unroll
     for (int q = 0; q < ROWS; ++q) {
-      const T p0 = P[q][0];
-      const T l = act[q] ? p0 * rpiv : T(0);
-#pragma unroll
-      for (int c = 0; c + 1 < W; ++c) P[q][c] = P[q][c + 1] - l * urow[j + 1 + c];
-      P[q][W - 1] = act[q] ? l : p0;
+      if ((int)rb + tid + q * NT == wi) won[q] = j;
+      l[q] = won[q] == W ? P[q][0] * rpiv : T(0);
+      top[q] = won[q] == W ? l[q] : P[q][0];
     }
+#pragma unroll
+    for (int c = 0; c + 1 < W; ++c) {
+      // bounds the row entries held in registers ahead of their use
+      if (c % kChunk == kChunk - 1) asm volatile("" ::: "memory");
+      const T uc = urow[1 + c];
+#pragma unroll
+      for (int q = 0; q < ROWS; ++q) P[q][c] = P[q][c + 1] - l[q] * uc;
+    }
+#pragma unroll
+    for (int q = 0; q < ROWS; ++q) P[q][W - 1] = top[q];
   }
   // the remaining rotations bring the columns back into register order
   for (int j = w; j < W; ++j) rotate();
 
-  // Replay the interchanges (LAPACK order: at step j rows at positions j and
-  // pos(winner) swap) to find every row's final position; wave 0 only.
+  // Replay the interchanges (LAPACK order: at step j the rows at position j
+  // and at the winner's position swap) to find every row's final position.
+  // Only two kinds of row move: the leaf's first w rows, and winners from
+  // below, each from its own place straight to its final position.  So lane
+  // r of wave 0 keeps the position of row r and the row at position r.
   if (tid < 64) {
-    if (tid == 0) ml.cnt = 0;
-    wave_sync();
+    const int win = lane < w ? s_win[lane] : 0;
+    int pos = lane, occ = lane, from = 0;
     for (int j = 0; j < w; ++j) {
-      const int64_t p = s_win[j];
-      const int cnt = ml.cnt;
-      const int ip = ml_find(ml.phys, cnt, p);
-      const int64_t pp = ip >= 0 ? ml.pos[ip] : p;         // position of the winner
-      const int iq = ml_find(ml.pos, cnt, (int64_t)j);
-      const int64_t q = iq >= 0 ? ml.phys[iq] : (int64_t)j; // row at position j
-      if (tid == 0) {
-        int k = ip;
-        if (k < 0) {
-          k = ml.cnt++;
-          ml.phys[k] = p;
-        }
-        ml.pos[k] = j;
-        if (q != p) {
-          // no listed row at position j means its occupant is row j itself,
-          // which is then not listed either
-          int kq = iq;
-          if (kq < 0) {
-            kq = ml.cnt++;
-            ml.phys[kq] = q;
-          }
-          ml.pos[kq] = pp;
-        }
-        if (g == 0) {
-          a.ipiv[j] = a.r0 + pp;
-          if (s_zero[j] && *a.info == 0) *a.info = (int32_t)(a.r0 + j + 1);
-        }
-      }
-      wave_sync();
+      const int p = __builtin_amdgcn_readlane(win, j);
+      const int pp = p < w ? __builtin_amdgcn_readlane(pos, p) : p;  // position of the winner
+      const int q = __builtin_amdgcn_readlane(occ, j);               // row at position j
+      if (lane == q) pos = pp;
+      if (lane == pp) occ = q;
+      if (lane == p) pos = j;
+      if (lane == j) from = pp;
+    }
+    if (lane < w) s_pos[lane] = pos;
+    const bool m1 = lane < w && pos != lane, m2 = lane < w && win >= w;
+    const unsigned long long b1 = __ballot(m1), b2 = __ballot(m2);
+    const unsigned long long below = (1ull << lane) - 1;
+    if (m1) {
+      const int k = __popcll(b1 & below);
+      ml.phys[k] = lane;
+      ml.pos[k] = pos;
+    }
+    if (m2) {
+      const int k = __popcll(b1) + __popcll(b2 & below);
+      ml.phys[k] = win;
+      ml.pos[k] = lane;
+    }
+    const unsigned long long z = __ballot(lane < w && s_zero[lane]);
+    if (lane == 0) ml.cnt = __popcll(b1) + __popcll(b2);
+    if (g == 0) {
+      if (lane < w) a.ipiv[lane] = a.r0 + from;
+      if (lane == 0 && z && *a.info == 0) *a.info = (int32_t)(a.r0 + __ffsll((long long)z));
     }
   }
   __syncthreads();
-  // every row of this workgroup to its final position
+  // every row of this workgroup to its final position (the bound is hidden
+  // from the compiler, which would keep the W column masks of the loads
+  // alive in scalar registers until here)
   const int cnt = ml.cnt;
+  int wst = w;
+  asm volatile("" : "+s"(wst));
 #pragma unroll
   for (int q = 0; q < ROWS; ++q) {
-    const int local = tid + q * kPanelThreads;
+    const int local = tid + q * NT;
     if (local >= nr) continue;
-    int64_t dest = rb + local;
-    for (int k = 0; k < cnt; ++k)
-      if (ml.phys[k] == rb + local) {
-        dest = ml.pos[k];
-        break;
-      }
+    const int64_t row = rb + local;
+    const int64_t dest = won[q] < W ? won[q] : row < w ? s_pos[row] : row;
     T* dst = a.A + dest * a.lda;
+    if (wide) {
 #pragma unroll
-    for (int c = 0; c < W; ++c)
-      if (c < w) dst[c] = P[q][c];
+      for (int c = 0; c < W; c += E) {
+        vec_t x;
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] = P[q][c + e];
+        *reinterpret_cast<vec_t*>(dst + c) = x;
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < W; ++c)
+        if (c < wst) dst[c] = P[q][c];
+    }
   }
   // The same interchanges on the outer panel's other columns (left and right
   // of this leaf), so the recursion above needs no row swaps of its own.
@@ -798,18 +941,18 @@ __global__ __launch_bounds__(kPanelThreads) void panel_kernel(PanelArgs<T> a) {
   const int64_t chunk = kSwapStage / cnt;  // columns per pass that fit the stage
   for (int64_t c0 = o0; c0 < o1; c0 += chunk) {
     const int64_t nc = c0 + chunk < o1 ? chunk : o1 - c0;
-    for (int64_t e = tid; e < (int64_t)cnt * nc; e += kPanelThreads) {
+    for (int64_t e = tid; e < (int64_t)cnt * nc; e += NT) {
       const int k = (int)(e / nc);
       const int64_t oc = c0 + e % nc;
       const int64_t col = oc < a.left ? oc - a.left : oc - a.left + w;
-      stage[e] = a.A[ml.phys[k] * a.lda + col];
+      stage[e] = a.A[(int64_t)ml.phys[k] * a.lda + col];
     }
     __syncthreads();
-    for (int64_t e = tid; e < (int64_t)cnt * nc; e += kPanelThreads) {
+    for (int64_t e = tid; e < (int64_t)cnt * nc; e += NT) {
       const int k = (int)(e / nc);
       const int64_t oc = c0 + e % nc;
       const int64_t col = oc < a.left ? oc - a.left : oc - a.left + w;
-      a.A[ml.pos[k] * a.lda + col] = stage[e];
+      a.A[(int64_t)ml.pos[k] * a.lda + col] = stage[e];
     }
     __syncthreads();
   }
@@ -1053,7 +1196,7 @@ struct LuCtx {
   hipStream_t s;
   // workspace
   double* cand;     // [2][G_max] (|value|, row) records of the panel launches
-  T* cand_row;      // [2][G_max][kPanelWMax]
+  unsigned long long* cand_row;  // [2][kKeyMaxGroups][kRowStride<T>]
   int* status;
   unsigned seq;     // steps taken by the panel launches so far
   LuScratch<T> sc;
@@ -1067,6 +1210,30 @@ struct LuCtx {
 // Upper bound on the workgroups of one leaf launch (0: the CU count).
 static std::atomic<int> g_panel_groups{0};
 constexpr int kPanelMaxRows = 3;  // rows per thread of the register-resident leaf
+
+// A leaf short enough for one workgroup of up to 1024 (FP32) or 768 (FP64)
+// rows, as many as its registers hold with one row per thread, is factored
+// by that workgroup alone: no exchange.  All leaves of an n x n LU, one
+// workgroup against 256-row workgroups: FP64 n = 512 1.75 / 1.90 ms, n = 768
+// 2.52 / 2.62 ms; FP32 n = 450 1.29 / 1.39 ms, n = 1024 3.10 / 3.49 ms.
+template <typename T>
+static bool lone_leaf(int64_t m, int w, int& nt, LeafShape& shape) {
+  static const struct { int nt, rows; } f64[] = {{kPanelThreads, 1}, {512, 1}, {768, 1}};
+  static const struct { int nt, rows; } f32[] = {{kPanelThreads, 1}, {512, 1}, {1024, 1}};
+  auto pick = [&](const auto& table) {
+    for (const auto& e : table)
+      if (m <= (int64_t)e.nt * e.rows) {
+        nt = e.nt;
+        shape.rows = e.rows;
+        shape.G = 1;
+        shape.R = m;
+        return true;
+      }
+    return false;
+  };
+  if (w <= kPanelWNarrow && m > kPanelThreads) return false;
+  return sizeof(T) == 8 ? pick(f64) : pick(f32);
+}
 
 template <typename T>
 static int leaf(LuCtx<T>& c, int64_t r0, int w) {
@@ -1086,8 +1253,12 @@ static int leaf(LuCtx<T>& c, int64_t r0, int w) {
   // As few workgroups as one row per thread allows (every column's exchange
   // polls all G records); more rows per thread only when the CUs run out.
   LeafShape shape;
-  RBFX_REQUIRE(leaf_shape(m, gmax, kPanelThreads, kPanelMaxRows, shape),
-               "matrix too large for the register-resident panel (m=%lld)", (long long)m);
+  // (a cap on the workgroups asks for the geometry below)
+  int nt = kPanelThreads;
+  if (!(g_panel_groups.load(std::memory_order_relaxed) == 0 && lone_leaf<T>(m, w, nt, shape))) {
+    RBFX_REQUIRE(leaf_shape(m, gmax, nt, kPanelMaxRows, shape),
+                 "matrix too large for the register-resident panel (m=%lld)", (long long)m);
+  }
   const int rows = shape.rows;
   const int G = shape.G;
   const int64_t R = shape.R;
@@ -1109,7 +1280,7 @@ static int leaf(LuCtx<T>& c, int64_t r0, int w) {
   a.status = c.status;
   a.info = c.info;
   a.wait_ticks = di.wait_ticks;
-  RBFX_REQUIRE(G <= c.G_max && G < kKeyMaxGroups && R <= (int64_t)kPanelThreads * rows && R < kKeyMaxRows,
+  RBFX_REQUIRE(G <= c.G_max && G < kKeyMaxGroups && R <= (int64_t)nt * rows && R < kKeyMaxRows,
                "too many panel workgroups or rows");
   const int pid = prof_start(sizeof(T) == 8 ? "panel_f64" : "panel_f32", c.s);
   // A plain launch on the panel stream.  The workgroups wait for each
@@ -1119,21 +1290,26 @@ static int leaf(LuCtx<T>& c, int64_t r0, int w) {
   // every wait is bounded in any case.  (A cooperative launch guarantees
   // the same but goes through a separate device queue, which added ~60 us
   // of dispatch latency per leaf, measured.)
-  if (w <= kPanelWNarrow) {
-    if (rows == 1)
-      hipLaunchKernelGGL((panel_kernel<T, 1, kPanelWNarrow>), dim3(G), dim3(kPanelThreads), 0, c.s, a);
-    else if (rows == 2)
-      hipLaunchKernelGGL((panel_kernel<T, 2, kPanelWNarrow>), dim3(G), dim3(kPanelThreads), 0, c.s, a);
-    else
-      hipLaunchKernelGGL((panel_kernel<T, 3, kPanelWNarrow>), dim3(G), dim3(kPanelThreads), 0, c.s, a);
+#define RBFX_LEAF(ROWS_, W_, NT_) \
+  hipLaunchKernelGGL((panel_kernel<T, ROWS_, W_, NT_>), dim3(G), dim3(NT_), 0, c.s, a)
+  if (nt != kPanelThreads) {
+    if (nt == 512 && rows == 1) RBFX_LEAF(1, kPanelWMax, 512);
+    else if (nt == 768 && rows == 1 && sizeof(T) == 8) RBFX_LEAF(1, kPanelWMax, sizeof(T) == 8 ? 768 : 512);
+    else if (nt == 1024 && rows == 1 && sizeof(T) == 4) RBFX_LEAF(1, kPanelWMax, sizeof(T) == 4 ? 1024 : 512);
+    else {
+      set_error("no leaf kernel of %d threads and %d rows per thread", nt, rows);
+      return RBFX_ERR_ARG;
+    }
+  } else if (w <= kPanelWNarrow) {
+    if (rows == 1) RBFX_LEAF(1, kPanelWNarrow, kPanelThreads);
+    else if (rows == 2) RBFX_LEAF(2, kPanelWNarrow, kPanelThreads);
+    else RBFX_LEAF(3, kPanelWNarrow, kPanelThreads);
   } else {
-    if (rows == 1)
-      hipLaunchKernelGGL((panel_kernel<T, 1, kPanelWMax>), dim3(G), dim3(kPanelThreads), 0, c.s, a);
-    else if (rows == 2)
-      hipLaunchKernelGGL((panel_kernel<T, 2, kPanelWMax>), dim3(G), dim3(kPanelThreads), 0, c.s, a);
-    else
-      hipLaunchKernelGGL((panel_kernel<T, 3, kPanelWMax>), dim3(G), dim3(kPanelThreads), 0, c.s, a);
+    if (rows == 1) RBFX_LEAF(1, kPanelWMax, kPanelThreads);
+    else if (rows == 2) RBFX_LEAF(2, kPanelWMax, kPanelThreads);
+    else RBFX_LEAF(3, kPanelWMax, kPanelThreads);
   }
+#undef RBFX_LEAF
   RBFX_CHECK_LAUNCH();
   prof_stop(pid, c.s, (double)m * w * w, 2.0 * sizeof(T) * m * w);
   c.seq += (unsigned)w;
@@ -1260,7 +1436,7 @@ static size_t getrf_ws_bytes(int64_t n, int bytes) {
   const int G = 1024;  // upper bound on workgroups of a leaf
   size_t b = 0;
   b += ws_round((size_t)2 * G * kRecWords * 8);   // cand records
-  b += ws_round((size_t)2 * G * kPanelWMax * bytes);  // cand_row
+  b += ws_round((size_t)2 * kKeyMaxGroups * (kPanelWMax + 2) * 2 * bytes);  // cand_row (tagged)
   b += ws_round(64);                              // status
   for (int q = 0; q < 3; ++q) {                   // two slots of the main stream, one of the panel stream
     b += ws_round((size_t)2 * kSwapMax * 8) * 2;  // plan dst / src
@@ -1354,7 +1530,8 @@ static int getrf(int64_t n, T* A, int64_t lda, int64_t* ipiv, void* work, size_t
   Workspace ws(work, work_bytes);
   const int G = 1024;
   c.cand = ws.take<double>((size_t)2 * G * kRecWords);
-  c.cand_row = ws.take<T>((size_t)2 * G * kPanelWMax);
+  constexpr size_t row_words = (size_t)2 * kKeyMaxGroups * kRowStride<T>;
+  c.cand_row = ws.take<unsigned long long>(row_words);
   unsigned* ctl = ws.take<unsigned>(16);
   c.status = reinterpret_cast<int*>(ctl + 1);
   // main stream: two slots of (plan, inverse) filled by the panel stream
@@ -1370,9 +1547,12 @@ static int getrf(int64_t n, T* A, int64_t lda, int64_t* ipiv, void* work, size_t
   c.G_max = G;
   hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, ctl, 16);
   RBFX_CHECK_LAUNCH();
-  // pivot records start with tag 0, which no column uses
+  // pivot records and candidate rows start with tag 0, which no column uses
   hipLaunchKernelGGL(zero_u32_kernel, dim3(4 * G * kRecWords / 64), dim3(64), 0, s,
                      reinterpret_cast<unsigned*>(c.cand), 4 * G * kRecWords);
+  RBFX_CHECK_LAUNCH();
+  hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)(2 * row_words / 256)), dim3(256), 0, s,
+                     reinterpret_cast<unsigned*>(c.cand_row), (int)(2 * row_words));
   RBFX_CHECK_LAUNCH();
   hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, reinterpret_cast<unsigned*>(info), 1);
   RBFX_CHECK_LAUNCH();
