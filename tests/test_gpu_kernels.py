@@ -143,6 +143,40 @@ def test_getrf_getrs(dtype, n):
 
 
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [1, 63, 65, 511, 513, 1100])
+def test_getrs_prepare_inverts_diagonal_blocks(dtype, n):
+    """The 64 x 64 and 512 x 512 inverses of the diagonal blocks of L and U
+    (identity past n) and their condition estimates, from the stored factors
+    of a diagonally dominant matrix (blocks of condition below 10)."""
+    from updes_amd import engine as E
+    _lib()
+    a = _random_well(n, n) + 4.0 * n * np.eye(n)
+    m = torch.zeros((n, E._ld(n)), dtype=dtype)
+    m[:, :n] = torch.as_tensor(a).to(dtype)
+    lu = E.LU(m.cuda(), n)
+    LU = lu.a[:, :n].double().cpu().numpy()
+    d = lu.dinv.cpu().numpy()
+    n64, n512 = -(-n // 64), -(-n // 512)
+    cond = d[n64 * 2 * 64 ** 2 + n512 * 2 * 512 ** 2:][:2 * n512].reshape(n512, 2)
+    off = 0
+    for size, count in ((64, n64), (512, n512)):
+        X = d[off:off + count * 2 * size ** 2].reshape(count, 2, size, size)
+        off += count * 2 * size ** 2
+        for b in range(count):
+            s = slice(b * size, min(n, (b + 1) * size))
+            w = s.stop - s.start
+            for which, T in ((0, np.tril(LU[s, s], -1) + np.eye(w)), (1, np.triu(LU[s, s]))):
+                full = np.eye(size)
+                full[:w, :w] = T
+                # each entry sums at most 512 products of a well-conditioned block
+                assert np.abs(X[b, which] @ full - np.eye(size)).max() <= 512 * 4 * np.finfo(float).eps * 10
+                if size == 512:
+                    Xw = X[b, which][:w, :w]
+                    ref = max(np.linalg.norm(T, p) * np.linalg.norm(Xw, p) for p in (1, np.inf))
+                    assert abs(cond[b, which] - ref) <= 1e-12 * ref
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("n", [511, 1301, 2100, 4099])
 def test_getrs_applies_stored_factors(dtype, n):
     """The superblock sweeps apply the stored factors (FP32 ones included) in

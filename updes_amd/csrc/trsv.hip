@@ -28,41 +28,57 @@ __host__ __device__ inline int64_t imin64(int64_t a, int64_t b) { return a < b ?
 
 // ---- diagonal-block inverses ----------------------------------------------
 // dinv[b][0] = inv(unit lower L_bb), dinv[b][1] = inv(U_bb), TB x TB row-major,
-// identity-padded for the last partial block.
-template <typename TF>
-__global__ __launch_bounds__(TB) void diag_inv_kernel(const TF* __restrict__ LU, int64_t lda, int64_t n,
-                                                      double* __restrict__ dinv) {
+// identity-padded for the last partial block.  One wave per (block,
+// triangle): lane c substitutes column c in registers (the loops unroll
+// fully), the block's entries are LDS broadcasts.  Bound by the dependent
+// chains of 2,016 FMAs and, for U, 64 divides.  At n = 603 this took 112 us
+// when both triangles were substituted through LDS by one wave.
+template <typename TF, int WHICH>
+__device__ __forceinline__ void diag_inv_body(const TF* __restrict__ LU, int64_t lda, int64_t n, int64_t b,
+                                              double (*S)[TB + 2], double* __restrict__ dinv) {
   typedef double T;
-  __shared__ T S[TB][TB + 1];
-  __shared__ T X[TB][TB + 1];
-  const int64_t b = blockIdx.x;
   const int64_t o = b * TB;
   const int sz = (int)imin64(TB, n - o);
   const int c = threadIdx.x;
+#pragma unroll 16
   for (int i = 0; i < TB; ++i) S[i][c] = (i < sz && c < sz) ? (T)LU[(o + i) * lda + o + c] : (i == c ? T(1) : T(0));
   __syncthreads();
-  // L^-1 column c: x_i = -sum_{c<=k<i} L_ik x_k
-  for (int i = 0; i < TB; ++i) X[i][c] = (i == c) ? T(1) : T(0);
-  for (int i = c + 1; i < TB; ++i) {
-    T s = 0;
-    for (int k = c; k < i; ++k) s += S[i][k] * X[k][c];
-    X[i][c] = (i < sz) ? -s : T(0);
-  }
-  T* Li = dinv + (b * 2) * TB * TB;
-  for (int i = 0; i < TB; ++i) Li[i * TB + c] = X[i][c];
-  __syncthreads();
-  // U^-1 column c: x_i = (delta_ic - sum_{k>i} U_ik x_k) / U_ii
-  for (int i = TB - 1; i >= 0; --i) {
-    if (i > c) {
-      X[i][c] = T(0);
-      continue;
+  T x[TB];
+  if constexpr (WHICH == 0) {
+    // L^-1 column c: x_i = -sum_{c<=k<i} L_ik x_k
+#pragma unroll
+    for (int i = 0; i < TB; ++i) {
+      T s = 0;
+#pragma unroll
+      for (int k = 0; k < i; ++k)
+        if (k >= c) s = __builtin_fma(S[i][k], x[k], s);
+      x[i] = i == c ? T(1) : (i > c && i < sz) ? -s : T(0);
     }
-    T s = (i == c) ? T(1) : T(0);
-    for (int k = i + 1; k <= c; ++k) s -= S[i][k] * X[k][c];
-    X[i][c] = s / S[i][i];
+  } else {
+    // U^-1 column c: x_i = (delta_ic - sum_{k>i} U_ik x_k) / U_ii
+#pragma unroll
+    for (int i = TB - 1; i >= 0; --i) {
+      T s = i == c ? T(1) : T(0);
+#pragma unroll
+      for (int k = i + 1; k < TB; ++k)
+        if (k <= c) s = __builtin_fma(-S[i][k], x[k], s);
+      x[i] = i > c ? T(0) : s / S[i][i];
+    }
   }
-  T* Ui = dinv + (b * 2 + 1) * TB * TB;
-  for (int i = 0; i < TB; ++i) Ui[i * TB + c] = X[i][c];
+  T* Xo = dinv + (b * 2 + WHICH) * TB * TB;
+#pragma unroll
+  for (int i = 0; i < TB; ++i) Xo[i * TB + c] = x[i];
+}
+
+template <typename TF>
+__global__ __launch_bounds__(TB) void diag_inv_kernel(const TF* __restrict__ LU, int64_t lda, int64_t n,
+                                                      double* __restrict__ dinv) {
+  __shared__ __align__(16) double S[TB][TB + 2];
+  const int64_t b = blockIdx.x >> 1;
+  if (blockIdx.x & 1)
+    diag_inv_body<TF, 1>(LU, lda, n, b, S, dinv);
+  else
+    diag_inv_body<TF, 0>(LU, lda, n, b, S, dinv);
 }
 
 // ---- permutation staging ------------------------------------------------------
@@ -117,98 +133,108 @@ constexpr int kCtlLine = 32;  // words per superblock control line
 // U (which = 1) in FP64, from the 64 x 64 inverses D_i of its sub-blocks:
 //   lower:  X_ii = D_i,  X_ij = -D_i sum_{j<=k<i} L_ik X_kj   (i > j)
 //   upper:  X_ii = D_i,  X_ij = -D_i sum_{i<k<=j} U_ik X_kj   (i < j)
-// One workgroup per (superblock, triangle); 64 x 64 tile products through
-// LDS, each thread a 4 x 4 block of the tile.  Rows and columns past n are
-// identity.
+// Columns of the inverse do not depend on each other, so a workgroup takes
+// kInvCols columns of one 64-wide block column: the chain is at most 35
+// products of a 64 x 64 tile with 64 x kInvCols values, kept in LDS, the next
+// tile loading meanwhile.  Each thread sums a 2 x 2 patch in a fixed order.
+// Rows and columns past n are identity.  With one workgroup per (superblock,
+// triangle) doing all 112 products through memory this took 1.31 ms at
+// n = 603 and 1.52 ms at n = 10,006.
+constexpr int kInvCols = 16;
+constexpr int kInvParts = TB / kInvCols;
 template <typename TF>
 __global__ __launch_bounds__(256) void sbinv_kernel(const TF* __restrict__ LU, int64_t lda, int64_t n,
                                                     const double* __restrict__ dinv64, double* __restrict__ dinv512) {
-  __shared__ double As[TB][TB + 1];
-  __shared__ double Bs[TB][TB + 1];
-  const int64_t K = blockIdx.x >> 1;
-  const int which = blockIdx.x & 1;
+  constexpr int NSUB = SB / TB;
+  constexpr int LX = kInvCols + 2;
+  typedef double vd2 __attribute__((ext_vector_type(2)));
+  __shared__ __align__(16) double Xs[SB][LX];  // the inverse's columns
+  __shared__ __align__(16) double Ts[TB][LX];
+  __shared__ __align__(16) double As[TB][TB + 2];
+  const int part = blockIdx.x % kInvParts;
+  const int j = (blockIdx.x / kInvParts) % NSUB;
+  const int which = (blockIdx.x / (kInvParts * NSUB)) & 1;
+  const int64_t K = blockIdx.x / (2 * kInvParts * NSUB);
   const int64_t o = K * SB;
   const int sz = (int)imin64(SB, n - o);
   const int nb = (sz + TB - 1) / TB;
-  constexpr int NSUB = SB / TB;
-  double* X = dinv512 + (K * 2 + which) * (int64_t)SB * SB;
+  const double* D64 = dinv64 + ((o / TB) * 2 + which) * TB * TB;  // of sub-block b: D64 + 2 b TB^2
   const int tid = threadIdx.x;
-  const int tr = (tid >> 4) * 4, tc = (tid & 15) * 4;
-  // X = blockdiag(D_i), identity past the matrix
-  for (int64_t e = tid; e < (int64_t)SB * SB; e += 256) {
-    const int r = (int)(e / SB), c = (int)(e % SB);
-    const int bi = r / TB, bj = c / TB;
+  const int r0 = (tid >> 3) * 2, c0 = (tid & 7) * 2;
+  const int lr = tid >> 6, lc = tid & 63;  // tile loads: rows lr + 4t, column lc
+  // column block j: D_j, identity past the matrix
+  for (int e = tid; e < SB * kInvCols; e += 256) {
+    const int r = e / kInvCols, c = e % kInvCols;
     double v = 0.0;
-    if (bi == bj) {
-      if (bi < nb)
-        v = dinv64[((o / TB + bi) * 2 + which) * TB * TB + (r % TB) * TB + (c % TB)];
-      else
-        v = r == c ? 1.0 : 0.0;
-    }
-    X[e] = v;
+    if (r / TB == j)
+      v = j < nb ? D64[(int64_t)j * 2 * TB * TB + (r % TB) * TB + part * kInvCols + c]
+                 : (r % TB == part * kInvCols + c ? 1.0 : 0.0);
+    Xs[r][c] = v;
   }
-  __syncthreads();
-  double acc[4][4];
-  auto tile_mma = [&](double sign) {
+  // The products in order: for each row block i away from the diagonal, the
+  // tiles (i, k) of the factor with the blocks k between j and i, then D_i.
+  // lower: rows below j; upper: rows above j, nearest first
+  const int steps = j >= nb ? 0 : which == 0 ? nb - 1 - j : j;
+  double ra[TB / 4];
+  auto load_tile = [&](int step, int kk) {
+    const int i = which == 0 ? j + step : j - step;
+    if (kk < step) {
+      // strictly lower / upper tile (i, k): no diagonal
+      const int k = which == 0 ? j + kk : i + 1 + kk;
 #pragma unroll
-    for (int q = 0; q < TB; ++q) {
-      double a[4], b[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        a[u] = As[tr + u][q];
-        b[u] = Bs[q][tc + u];
+      for (int t = 0; t < TB / 4; ++t) {
+        const int gr = i * TB + lr + 4 * t, gc = k * TB + lc;
+        ra[t] = (gr < sz && gc < sz) ? (double)LU[(o + gr) * lda + o + gc] : 0.0;
       }
+    } else {
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] = __builtin_fma(sign * a[u], b[v], acc[u][v]);
+      for (int t = 0; t < TB / 4; ++t) ra[t] = D64[(int64_t)i * 2 * TB * TB + (lr + 4 * t) * TB + lc];
     }
   };
-  for (int j = 0; j < nb; ++j) {
-    for (int step = 1; step < nb; ++step) {
-      // lower: rows below j; upper: rows above j, nearest first
-      const int i = which == 0 ? j + step : j - step;
-      if (i < 0 || i >= nb) break;
+  if (steps > 0) load_tile(1, 0);
+  for (int step = 1; step <= steps; ++step) {
+    const int i = which == 0 ? j + step : j - step;
+    double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
+    for (int kk = 0; kk <= step; ++kk) {
+      __syncthreads();  // As free, Xs / Ts written
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+      for (int t = 0; t < TB / 4; ++t) As[lr + 4 * t][lc] = ra[t];
+      __syncthreads();
+      if (kk < step)
+        load_tile(step, kk + 1);
+      else if (step < steps)
+        load_tile(step + 1, 0);
+      const bool last = kk == step;  // X_ij = -D_i T
+      const double* B = last ? &Ts[0][0] : &Xs[(which == 0 ? j + kk : i + 1 + kk) * TB][0];
+      const double sign = last ? -1.0 : 1.0;
+#pragma unroll 8
+      for (int q = 0; q < TB; q += 2) {
+        vd2 a[2];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] = 0.0;
-      const int k0 = which == 0 ? j : i + 1, k1 = which == 0 ? i - 1 : j;
-      for (int k = k0; k <= k1; ++k) {
-        // As = factor tile (i, k) (strictly lower / upper: no diagonal), Bs = X tile (k, j)
-        for (int e = tid; e < TB * TB; e += 256) {
-          const int r = e / TB, c = e % TB;
-          const int gr = i * TB + r, gc = k * TB + c;
-          As[r][c] = (gr < sz && gc < sz) ? (double)LU[(o + gr) * lda + o + gc] : 0.0;
-          Bs[r][c] = X[(int64_t)(k * TB + r) * SB + j * TB + c];
+        for (int u = 0; u < 2; ++u) a[u] = *reinterpret_cast<const vd2*>(&As[r0 + u][q]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const vd2 b = *reinterpret_cast<const vd2*>(B + (q + h) * LX + c0);
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            acc[u][0] = __builtin_fma(sign * a[u][h], b.x, acc[u][0]);
+            acc[u][1] = __builtin_fma(sign * a[u][h], b.y, acc[u][1]);
+          }
         }
-        __syncthreads();
-        tile_mma(1.0);
-        __syncthreads();
       }
-      // X_ij = -D_i T: As = D_i, Bs = T
-      for (int e = tid; e < TB * TB; e += 256) {
-        const int r = e / TB, c = e % TB;
-        As[r][c] = X[(int64_t)(i * TB + r) * SB + i * TB + c];
+      if (kk >= step - 1) {
+        double* dst = last ? &Xs[i * TB][0] : &Ts[0][0];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          *reinterpret_cast<vd2*>(dst + (r0 + u) * LX + c0) = vd2{acc[u][0], acc[u][1]};
+          acc[u][0] = acc[u][1] = 0.0;
+        }
       }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) Bs[tr + u][tc + v] = acc[u][v];
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] = 0.0;
-      tile_mma(-1.0);
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) X[(int64_t)(i * TB + tr + u) * SB + j * TB + tc + v] = acc[u][v];
-      __syncthreads();
     }
   }
-  (void)NSUB;
+  __syncthreads();
+  double* X = dinv512 + (K * 2 + which) * (int64_t)SB * SB + j * TB + part * kInvCols;
+  for (int e = tid; e < SB * kInvCols; e += 256) X[(int64_t)(e / kInvCols) * SB + e % kInvCols] = Xs[e / kInvCols][e % kInvCols];
 }
 
 // Condition estimate of every diagonal superblock T_KK of L (which = 0, unit
@@ -217,47 +243,86 @@ __global__ __launch_bounds__(256) void sbinv_kernel(const TF* __restrict__ LU, i
 // kCondRobust; above it they solve the block by substitution over its 64-row
 // sub-blocks (one refinement step with X reduces the block residual by about
 // kappa eps, so X serves a backward-stable solve only for kappa well below
-// eps^-1/2).
+// eps^-1/2).  kCondParts workgroups per (superblock, triangle) sum 64 rows
+// and 64 columns each (coalesced: a wave per row, a lane per column), then
+// one thread combines the parts.  0.49 ms at n = 603 when one workgroup
+// summed a row and a column per thread.
 constexpr double kCondRobust = 1e7;
+constexpr int kCondParts = SB / 64;
+constexpr int kCondThreads = 512;
 template <typename TF>
-__global__ __launch_bounds__(256) void sbcond_kernel(const TF* __restrict__ LU, int64_t lda, int64_t n,
-                                                     const double* __restrict__ dinv512, double* __restrict__ cond) {
-  __shared__ double red[4][256];
-  const int I = blockIdx.x >> 1, which = blockIdx.x & 1;
-  const int64_t o = (int64_t)I * SB;
+__global__ __launch_bounds__(kCondThreads) void sbcond_part_kernel(const TF* __restrict__ LU, int64_t lda, int64_t n,
+                                                                   const double* __restrict__ dinv512,
+                                                                   double* __restrict__ part) {
+  constexpr int NW = kCondThreads / 64;
+  __shared__ double rows[2][NW], cols[2][NW][64];
+  const int64_t blk = blockIdx.x / kCondParts;
+  const int p0 = (int)(blockIdx.x % kCondParts) * 64;
+  const int64_t I = blk >> 1;
+  const int which = (int)(blk & 1);
+  const int64_t o = I * SB;
   const int sz = (int)imin64(SB, n - o);
-  const double* X = dinv512 + (int64_t)blockIdx.x * SB * SB;
-  double tr = 0, tc = 0, xr = 0, xc = 0;  // max row / column sums of |T| and |X|
-  for (int q = threadIdx.x; q < sz; q += 256) {
-    double a = 0, b = 0, cx = 0, dx = 0;
-    for (int k = 0; k < sz; ++k) {
-      // row q and column q of the triangle (unit diagonal for L)
-      const bool inr = which ? k >= q : k < q;
-      const bool inc = which ? k <= q : k > q;
-      if (inr) a += fabs((double)LU[(o + q) * lda + o + k]);
-      if (inc) b += fabs((double)LU[(o + k) * lda + o + q]);
-      cx += fabs(X[(int64_t)q * SB + k]);
-      dx += fabs(X[(int64_t)k * SB + q]);
+  const double* X = dinv512 + blk * (int64_t)SB * SB;
+  const TF* F = LU + o * lda + o;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  auto entry = [&](int r, int c) -> double {  // |T[r][c]| (unit diagonal for L)
+    if (which ? c < r : c > r) return 0.0;
+    return which == 0 && c == r ? 1.0 : fabs((double)F[(int64_t)r * lda + c]);
+  };
+  double tr = 0, xr = 0;  // largest row sums of this wave
+  for (int r = p0 + w; r < p0 + 64 && r < sz; r += NW) {
+    double a = 0, x = 0;
+#pragma unroll
+    for (int t = 0; t < SB / 64; ++t) {
+      const int c = lane + 64 * t;
+      if (c < sz) {
+        a += entry(r, c);
+        x += fabs(X[(int64_t)r * SB + c]);
+      }
     }
-    if (!which) {
-      a += 1.0;
-      b += 1.0;
+    for (int off = 32; off > 0; off >>= 1) {
+      a += __shfl_xor(a, off, 64);
+      x += __shfl_xor(x, off, 64);
     }
     tr = fmax(tr, a);
-    tc = fmax(tc, b);
-    xr = fmax(xr, cx);
-    xc = fmax(xc, dx);
+    xr = fmax(xr, x);
   }
-  red[0][threadIdx.x] = tr;
-  red[1][threadIdx.x] = tc;
-  red[2][threadIdx.x] = xr;
-  red[3][threadIdx.x] = xc;
+  if (lane == 0) {
+    rows[0][w] = tr;
+    rows[1][w] = xr;
+  }
+  double tc = 0, xc = 0;  // this lane's column, the rows w, w + NW, ...
+  const int c = p0 + lane;
+  if (c < sz)
+#pragma unroll 16
+    for (int r = w; r < sz; r += NW) {
+      tc += entry(r, c);
+      xc += fabs(X[(int64_t)r * SB + c]);
+    }
+  cols[0][w][lane] = tc;
+  cols[1][w][lane] = xc;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int t = 1; t < 256; ++t)
-      for (int e = 0; e < 4; ++e) red[e][0] = fmax(red[e][0], red[e][t]);
-    cond[blockIdx.x] = fmax(red[0][0] * red[2][0], red[1][0] * red[3][0]);
+  if (w < 2) {
+    double v = 0, m = 0;
+    for (int q = 0; q < NW; ++q) {
+      v += cols[w][q][lane];
+      m = fmax(m, rows[w][q]);
+    }
+    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+    if (lane == 0) {
+      part[blockIdx.x * 4 + 2 * w] = m;      // 0: T rows, 2: X rows
+      part[blockIdx.x * 4 + 2 * w + 1] = v;  // 1: T columns, 3: X columns
+    }
   }
+}
+
+__global__ void sbcond_kernel(int64_t nblk, const double* __restrict__ part, double* __restrict__ cond) {
+  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= nblk) return;
+  double m[4] = {0, 0, 0, 0};
+  for (int p = 0; p < kCondParts; ++p)
+    for (int e = 0; e < 4; ++e) m[e] = fmax(m[e], part[(b * kCondParts + p) * 4 + e]);
+  cond[b] = fmax(m[0] * m[2], m[1] * m[3]);
 }
 
 // ctl[0] ticket, ctl[1] superblocks solved, ctl[2] status of the solve; the
@@ -809,6 +874,22 @@ static int prepare(int64_t n, const T* LU, int64_t lda, const int64_t* ipiv, int
   std::vector<int64_t> hp(n), pm(n);
   RBFX_HIP(hipMemcpyAsync(hp.data(), ipiv, n * sizeof(int64_t), hipMemcpyDeviceToHost, s));
   RBFX_HIP(hipStreamSynchronize(s));
+  // the inverses run while the host replays the interchanges
+  const int64_t nsb = ceil_div(n, (int64_t)SB);
+  double* d512 = dinv + dinv64_elems(n);
+  double* cond = d512 + nsb * 2 * (int64_t)SB * SB;
+  double* part = cond + 2 * nsb;
+  hipLaunchKernelGGL((diag_inv_kernel<T>), dim3((unsigned)(2 * ceil_div(n, TB))), dim3(TB), 0, s, LU, lda, n, dinv);
+  RBFX_CHECK_LAUNCH();
+  hipLaunchKernelGGL((sbinv_kernel<T>), dim3((unsigned)(2 * nsb * (SB / TB) * kInvParts)), dim3(256), 0, s, LU, lda, n,
+                     (const double*)dinv, d512);
+  RBFX_CHECK_LAUNCH();
+  hipLaunchKernelGGL((sbcond_part_kernel<T>), dim3((unsigned)(2 * nsb * kCondParts)), dim3(kCondThreads), 0, s, LU, lda,
+                     n, (const double*)d512, part);
+  RBFX_CHECK_LAUNCH();
+  hipLaunchKernelGGL(sbcond_kernel, dim3((unsigned)ceil_div(2 * nsb, 256)), dim3(256), 0, s, 2 * nsb,
+                     (const double*)part, cond);
+  RBFX_CHECK_LAUNCH();
   for (int64_t i = 0; i < n; ++i) pm[i] = i;
   for (int64_t i = 0; i < n; ++i) {
     const int64_t p = hp[i];
@@ -816,16 +897,6 @@ static int prepare(int64_t n, const T* LU, int64_t lda, const int64_t* ipiv, int
     std::swap(pm[i], pm[p]);
   }
   RBFX_HIP(hipMemcpyAsync(perm, pm.data(), n * sizeof(int64_t), hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL((diag_inv_kernel<T>), dim3((unsigned)ceil_div(n, TB)), dim3(TB), 0, s, LU, lda, n, dinv);
-  RBFX_CHECK_LAUNCH();
-  const int64_t nsb = ceil_div(n, (int64_t)SB);
-  double* d512 = dinv + dinv64_elems(n);
-  hipLaunchKernelGGL((sbinv_kernel<T>), dim3((unsigned)(2 * nsb)), dim3(256), 0, s, LU, lda, n, (const double*)dinv,
-                     d512);
-  RBFX_CHECK_LAUNCH();
-  hipLaunchKernelGGL((sbcond_kernel<T>), dim3((unsigned)(2 * nsb)), dim3(256), 0, s, LU, lda, n, (const double*)d512,
-                     d512 + nsb * 2 * (int64_t)SB * SB);
-  RBFX_CHECK_LAUNCH();
   RBFX_HIP(hipStreamSynchronize(s));  // pm must outlive the copy
   return RBFX_OK;
 }
@@ -845,7 +916,7 @@ extern "C" int rbfx_getrs_multi_f64(int64_t n, const double* d_LU, int64_t lda, 
 }
 
 extern "C" int64_t rbfx_getrs_dinv_elems(int64_t n) {
-  return n <= 0 ? 0 : dinv64_elems(n) + ceil_div(n, (int64_t)SB) * (2 * (int64_t)SB * SB + 2);
+  return n <= 0 ? 0 : dinv64_elems(n) + ceil_div(n, (int64_t)SB) * (2 * (int64_t)SB * SB + 2 + 8 * kCondParts);
 }
 
 extern "C" size_t rbfx_getrs_workspace(int64_t n) {
