@@ -88,6 +88,31 @@ def test_gemm_matches_torch(dtype, m, n, k, beta):
     assert err < tol, err
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 16), (65, 3, 16), (130, 63, 32), (64, 65, 64), (300, 129, 64),
+                                   (2945, 2951, 32)])
+def test_gemm_ragged_columns_in_padded_rows(dtype, m, n, k):
+    """A column count that is not a whole number of 16-byte chunks, in rows
+    that hold the last chunk: same product, and the padding behind C's rows
+    stays as it was (B's padding is NaN and must not reach a result)."""
+    L = _lib()
+    ld = -(-n // 64) * 64
+    g = torch.Generator().manual_seed(m + n + k)
+    A = torch.randn(m, k, generator=g, dtype=torch.float64)
+    B = torch.full((k, ld), float("nan"), dtype=torch.float64)
+    B[:, :n] = torch.randn(k, n, generator=g, dtype=torch.float64)
+    C = torch.randn(m, ld, generator=g, dtype=torch.float64)
+    dA, dB, dC = (t.to(dtype).cuda().contiguous() for t in (A, B, C))
+    pad = dC[:, n:].clone()
+    ref = C[:, :n] - A @ B[:, :n]
+    fn = L.lib().rbfx_gemm_f64 if dtype == torch.float64 else L.lib().rbfx_gemm_f32
+    L.check(fn(m, n, k, -1.0, L.ptr(dA), k, L.ptr(dB), ld, 1.0, L.ptr(dC), ld, L.stream()))
+    torch.cuda.synchronize()
+    tol = 1e-12 if dtype == torch.float64 else 2e-4
+    assert (dC[:, :n].double().cpu() - ref).abs().max().item() < tol * max(1.0, ref.abs().max().item())
+    assert torch.equal(dC[:, n:], pad)
+
+
 @pytest.mark.parametrize("alpha", [0.5, 1.0])
 def test_gemm_alpha(alpha):
     """alpha = +-1 takes the LDS-DMA kernel, other values the register-staged one."""
@@ -257,6 +282,25 @@ def test_getrf_f32_leaf_geometry_does_not_change_the_factors():
     assert default.singular == 0 and wide.singular == 0
     assert torch.equal(default.ipiv, wide.ipiv)
     assert torch.equal(default.a[:, :n], wide.a[:, :n])
+
+
+@pytest.mark.parametrize("n", [4096, 4097, 4161, 4608])
+def test_getrf_f64_panels_at_the_recursion_limit(n):
+    """FP64 panels are recursive up to n = 4096 and factored leaf by leaf
+    above; last panels of 1, 65 and 512 columns.  Same pivots as LAPACK and the
+    P A - L U residual of a partial-pivoting LU."""
+    from updes_amd import engine as E
+    _lib()
+    a = _random_well(n, n)
+    m = torch.zeros((n, E._ld(n)), dtype=torch.float64)
+    m[:, :n] = torch.as_tensor(a)
+    lu = E.LU(m.cuda(), n)
+    assert lu.singular == 0
+    assert np.array_equal(lu.ipiv.cpu().numpy(), sla.lu_factor(a)[1])
+    LU = lu.a[:, :n]
+    PA = torch.as_tensor(a).cuda()[lu.perm]
+    R = (torch.tril(LU, -1) + torch.eye(n, dtype=torch.float64, device="cuda")) @ torch.triu(LU) - PA
+    assert R.abs().max().item() < 1e-13 * n * np.abs(a).max()
 
 
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])

@@ -224,8 +224,10 @@ __global__ __launch_bounds__(GTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
 // k = E g + s, so one 16-byte read gives a lane its A values of all E MFMAs.
 // For B one 16-byte read gives E adjacent columns, which feed E adjacent
 // n-tiles: tile j's column for lane column c is 16E (j/E) + E c + j%E.
-// Requirements (checked by the host): k % BK == 0, n % E == 0, lda, ldb and
-// ldc multiples of E, 16-byte aligned A, B and C.
+// Requirements (checked by the host): k % BK == 0, lda, ldb and ldc multiples
+// of E, 16-byte aligned A, B and C, and rows of B and C that hold the whole
+// last chunk (ld >= n rounded up to E): its columns past n are read, and only
+// those before n are stored.
 constexpr int kGemmStages = 4;
 
 // BT x BT block tile (BT = 128, or 64 for small FP64 products), 2 x 2 waves
@@ -268,7 +270,7 @@ __device__ __forceinline__ void gemm_dma_body(int64_t m, int64_t n, int64_t k, T
   const int lg = lane >> 4, lc = lane & 15;
 
   // DMA sources of this thread (RC A chunks, RC B chunks per k-tile); rows
-  // past m are clamped (their results are never stored)
+  // past m and chunks past n are clamped (their results are never stored)
   const T* srcA[RC];
   const T* srcB[RC];
 #pragma unroll
@@ -278,7 +280,7 @@ __device__ __forceinline__ void gemm_dma_body(int64_t m, int64_t n, int64_t k, T
     const int64_t row = row0 + mm < m ? row0 + mm : m - 1;
     srcA[r] = A + row * lda + g * E;
     const int kk = p / NG, q = p % NG;
-    const int64_t col = col0 + (int64_t)q * E < n ? col0 + (int64_t)q * E : n - E;
+    const int64_t col = col0 + (int64_t)q * E < n ? col0 + (int64_t)q * E : (n - 1) / E * E;
     srcB[r] = B + (int64_t)kk * ldb + col;
   }
   auto issue = [&](int64_t kt, int st) {
@@ -367,7 +369,11 @@ __device__ __forceinline__ void gemm_dma_body(int64_t m, int64_t n, int64_t k, T
         vec_t x;
 #pragma unroll
         for (int e = 0; e < E; ++e) x[e] = neg ? -acc[i][jg * E + e][v] : acc[i][jg * E + e][v];
-        *reinterpret_cast<vec_t*>(C + r * ldc + c) = x;
+        if (c + E <= n) {
+          *reinterpret_cast<vec_t*>(C + r * ldc + c) = x;
+        } else {
+          for (int e = 0; c + e < n; ++e) C[r * ldc + c + e] = x[e];
+        }
       }
     }
 }
@@ -396,14 +402,17 @@ __global__ __launch_bounds__(GTHREADS) void gemm_dma64_kernel(int64_t m, int64_t
 // fit beside two update workgroups on a CU instead of waiting for one to end.
 template <typename T, int USE = 0>
 static int gemm_launch(int64_t m, int64_t n, int64_t k, T alpha, const T* A, int64_t lda, const T* B,
-                       int64_t ldb, T beta, T* C, int64_t ldc, hipStream_t s, bool small_lds = false) {
+                       int64_t ldb, T beta, T* C, int64_t ldc, hipStream_t s, bool small_lds = false,
+                       bool ragged = true) {
   if (m <= 0 || n <= 0) return RBFX_OK;
   const int64_t tm = ceil_div(m, GBM), tn = ceil_div(n, GBN);
   const int64_t tiles = tm * tn;
   const int64_t grid = ((tiles + 7) / 8) * 8;
   constexpr int E = 16 / (int)sizeof(T);
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  const bool dma = (alpha == T(1) || alpha == T(-1)) && k > 0 && k % Mma<T>::BK == 0 && n >= E && n % E == 0 && lda % E == 0 && ldb % E == 0 &&
+  const bool dma = (alpha == T(1) || alpha == T(-1)) && k > 0 && k % Mma<T>::BK == 0 && (n % E == 0 || ragged) && n >= E &&
+                   ldb >= ceil_div(n, (int64_t)E) * E &&
+                   ldc >= ceil_div(n, (int64_t)E) * E && lda % E == 0 && ldb % E == 0 &&
                    ldc % E == 0 && al16(A) && al16(B) && al16(C);
   if (dma && sizeof(T) == 8 && tiles < 2 * (int64_t)device_info().num_cus) {
     const int64_t tm64 = ceil_div(m, (int64_t)64), tn64 = ceil_div(n, (int64_t)64);
@@ -426,19 +435,30 @@ static int gemm_launch(int64_t m, int64_t n, int64_t k, T alpha, const T* A, int
 
 template <typename T>
 static int gemm(int64_t m, int64_t n, int64_t k, T alpha, const T* A, int64_t lda, const T* B,
-                int64_t ldb, T beta, T* C, int64_t ldc, hipStream_t s, bool in_panel = false) {
+                int64_t ldb, T beta, T* C, int64_t ldc, hipStream_t s, bool in_panel = false, bool ragged = true) {
   if (m <= 0 || n <= 0) return RBFX_OK;
   // profile names: the trailing update of the factorisation (and direct
   // calls) vs the updates inside a recursive panel
   const int pid = prof_start(in_panel ? (sizeof(T) == 8 ? "gemm_panel_f64" : "gemm_panel_f32")
                                       : (sizeof(T) == 8 ? "gemm_f64" : "gemm_f32"),
                              s);
-  const int st = in_panel ? gemm_launch<T, 3>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s, true)
-                          : gemm_launch<T, 0>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s);
+  const int st = in_panel ? gemm_launch<T, 3>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s, true, ragged)
+                          : gemm_launch<T, 0>(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s, false, ragged);
   prof_stop(pid, s, 2.0 * m * n * k, (double)sizeof(T) * (2.0 * m * n + (double)m * k + (double)k * n));
   return st;
 }
 
+
+// Row block b (64 rows, the last one w) of the inverse X of an outer panel's
+// unit-lower diagonal block: X_b0 .. X_bb from the rows of L and X above.
+template <typename T>
+struct InvArgs {
+  const T* P = nullptr;  // first row and column of the outer panel
+  int64_t lda = 0;
+  T* X = nullptr;
+  int64_t ldx = 0;
+  int b = -1, w = 0;
+};
 
 template <typename T>
 struct PanelArgs {
@@ -448,7 +468,10 @@ struct PanelArgs {
   int w;          // panel width <= kPanelWMax
   int64_t R;      // rows per workgroup
   int64_t r0;     // absolute row of the panel's first row
-  int64_t left, right;  // columns of the enclosing outer panel left / right of the leaf
+  int G;          // workgroups of the leaf; the ones past it invert (below)
+  int* moves;     // [kMoveStride] out: the leaf's winners, final positions of its first rows, o and w
+  int o;          // first column of the leaf in its outer panel
+  InvArgs<T> inv; // a finished diagonal block whose rows of the panel's inverse ride along
   int64_t* ipiv;  // (w) absolute pivot rows
   double* cand;   // [2][G][kRecWords] tagged (|value|, row) records (first two words used)
   unsigned long long* cand_row;  // [2][G][kRowStride<T>] tagged words of the candidate rows
@@ -460,6 +483,7 @@ struct PanelArgs {
 
 constexpr int kPanelThreads = 256;     // leaf workgroups that run beside a trailing update
 constexpr int kPanelWMax = 64;
+constexpr int kMoveStride = 2 * kPanelWMax + 2;
 // A published row entry carries its own tag: each 64-bit word holds 32 bits
 // of the value and the 32-bit tag of its column, so a reader that finds the
 // tag has the value, and the writer need not wait between the row and the
@@ -469,18 +493,12 @@ constexpr int kRowWords = sizeof(T) / 4;
 // a published row: kPanelWMax entries and the reciprocal of the first
 template <typename T>
 constexpr int kRowStride = (kPanelWMax + 2) * kRowWords<T>;
-// Narrow leaves for the panels that run beside a long trailing update: a
-// 16-wide FP64 leaf (67 VGPRs) shares a CU with two trailing-update
-// workgroups (2 x 216 VGPRs per SIMD), where a 64-wide one (164) displaces
-// one of them.  More leaves and splits per panel, hidden under the update
-// while it is long: panels of at least kNarrowLeafRows rows (measured best
-// at n = 40,006 among 20k..36k).  FP32 only uses them on request: a 64-wide
-// FP32 leaf (95 VGPRs) already fits beside two update workgroups, and the
-// FP32 update is too short to hide the narrow leaves' extra launches
-// (40k mixed step: 615 ms without, 621 ms from 28,000 rows, 625 ms from
-// 20,000).
+// Narrow leaves, on request only (rbfx_set_narrow_leaf_rows): a 16-wide FP64
+// leaf (72 VGPRs) shares a CU with two trailing-update workgroups (2 x 216
+// VGPRs per SIMD), a 64-wide one (202) displaces one of them.  That paid when
+// a panel cost more than the update beside it; now an FP64 LU takes 832 ms with
+// them and 835 ms without at n = 40,006, 466 and 464 ms at n = 32,006.
 constexpr int kPanelWNarrow = 16;
-constexpr int64_t kNarrowLeafRows = 28000;
 static std::atomic<int64_t> g_narrow_leaf_rows{0};
 // A pivot record (two 64-bit words) owns a 128-byte line: every workgroup
 // polls every record, and records sharing a line would serialise the polls.
@@ -562,14 +580,6 @@ __device__ inline unsigned long long block_max_key(unsigned long long key, unsig
   }
 }
 
-// The rows that a leaf moves and their final positions (a row that is not
-// listed stays where it is).
-struct MoveList {
-  int phys[2 * kPanelWMax];
-  int pos[2 * kPanelWMax];
-  int cnt;
-};
-
 // Orders lane 0's LDS writes before the wave's following LDS reads.
 __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -577,8 +587,102 @@ __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Staging of the interchanges applied to the panel's other columns.
-constexpr int kSwapStage = 2048;
+// ---- small triangular solves on MFMA tiles ----------------------------------
+constexpr int kTri = 64;
+
+// One wave: the inverse of a 16 x 16 unit-lower block by forward
+// substitution, the solved row broadcast by lane shuffles; lane l ends with
+// rows 4q + l/16 of column l%16.  L(i, k) gives the entries below the diagonal.
+template <typename F>
+__device__ inline void tri_inv16(F&& L, double (*out)[17]) {
+  const int lane = threadIdx.x & 63, c = lane & 15, r4 = lane >> 4;
+  double y[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) y[q] = (4 * q + r4 == c) ? 1.0 : 0.0;
+#pragma unroll
+  for (int k = 0; k < 15; ++k) {
+    const double xk = __shfl(y[k >> 2], ((k & 3) << 4) | c, 64);  // X[k][c]
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = 4 * q + r4;
+      if (i > k) y[q] -= L(i, k) * xk;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) out[4 * q + r4][c] = y[q];
+}
+
+// One wave: acc (four 16 x 16 tiles, rows 16 I of 16 columns, accumulator
+// layout) <- inv(L) acc for the 64 x 64 unit-lower L, given its entries below
+// the 16 x 16 diagonal blocks and those blocks' inverses.  An accumulator
+// tile is the B operand of the next product as it stands: MFMA k-step s takes
+// row Mma<T>::row(lane, s), element s of the tile.
+template <typename T, typename F>
+__device__ inline void tri_solve64(typename Mma<T>::acc_t (&acc)[4], F&& L, const double (*inv)[16][17]) {
+  const int lane = threadIdx.x & 63, m = lane & 15;
+#pragma unroll
+  for (int I = 0; I < 4; ++I) {
+#pragma unroll
+    for (int J = 0; J < I; ++J)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        acc[I] = Mma<T>::mma(-L(16 * I + m, 16 * J + Mma<T>::row(lane, s)), acc[J][s], acc[I]);
+    typename Mma<T>::acc_t u = {};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) u = Mma<T>::mma((T)inv[I][m][Mma<T>::row(lane, s)], acc[I][s], u);
+    acc[I] = u;
+  }
+}
+
+// Columns 64 q .. of row block v.b of the inverse (q <= v.b), by four waves:
+// inv(L_bb) (-sum_{q <= k < b} L_bk X_kq), or inv(L_bb) itself for q = b.
+// Operands come straight from memory: it runs beside the next leaf, or once
+// at the panel's end.
+template <typename T>
+__device__ inline void inverse_rows(const InvArgs<T>& v, int q, double (*inv)[16][17]) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, m = lane & 15;
+  const T* Lb = v.P + (int64_t)kTri * v.b * v.lda;  // rows of the block
+  const T* D = Lb + kTri * v.b;
+  tri_inv16(
+      [&](int i, int k) -> double {
+        return 16 * wv + i < v.w ? (double)D[(int64_t)(16 * wv + i) * v.lda + 16 * wv + k] : 0.0;
+      },
+      inv[wv]);
+  __syncthreads();
+  typename Mma<T>::acc_t acc[4];
+#pragma unroll
+  for (int I = 0; I < 4; ++I)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      acc[I][e] = q == v.b && 16 * I + Mma<T>::row(lane, e) == 16 * wv + m ? T(1) : T(0);
+  const int c0 = kTri * q + 16 * wv + m;  // this lane's column of X
+  for (int k = q; k < v.b; ++k) {
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      T bv[4], av[4][4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int kk = kTri * k + 16 * kb + Mma<T>::row(lane, s);
+        bv[s] = v.X[(int64_t)kk * v.ldx + c0];
+#pragma unroll
+        for (int I = 0; I < 4; ++I) av[I][s] = 16 * I + m < v.w ? Lb[(int64_t)(16 * I + m) * v.lda + kk] : T(0);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int I = 0; I < 4; ++I) acc[I] = Mma<T>::mma(-av[I][s], bv[s], acc[I]);
+    }
+  }
+  tri_solve64<T>(
+      acc, [&](int i, int k) -> T { return i < v.w ? D[(int64_t)i * v.lda + k] : T(0); }, inv);
+#pragma unroll
+  for (int I = 0; I < 4; ++I)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 16 * I + Mma<T>::row(lane, e);
+      if (r < v.w && (q < v.b || 16 * wv + m < v.w)) v.X[(int64_t)(kTri * v.b + r) * v.ldx + c0] = acc[I][e];
+    }
+}
 
 // The W words of row q's candidate (tagged with tag) to lane c < n: entry c.
 template <typename T>
@@ -641,10 +745,16 @@ __global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {
   __shared__ int s_win[W];
   __shared__ int s_zero[W];
   __shared__ int s_pos[W];
-  __shared__ MoveList ml;
-  __shared__ T stage[kSwapStage];
 
-  const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x;
+  const int G = a.G, g = blockIdx.x, tid = threadIdx.x;
+  if constexpr (W > kPanelWNarrow) {
+    // rows of the panel's inverse that the leaf before made possible
+    if (g >= G) {
+      __shared__ double s_inv[4][16][17];
+      if (tid < 256) inverse_rows<T>(a.inv, g - G, s_inv);
+      return;
+    }
+  }
   const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int w = a.w;
   const int64_t rb = (int64_t)g * a.R;
@@ -881,23 +991,17 @@ __global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {
       if (lane == j) from = pp;
     }
     if (lane < w) s_pos[lane] = pos;
-    const bool m1 = lane < w && pos != lane, m2 = lane < w && win >= w;
-    const unsigned long long b1 = __ballot(m1), b2 = __ballot(m2);
-    const unsigned long long below = (1ull << lane) - 1;
-    if (m1) {
-      const int k = __popcll(b1 & below);
-      ml.phys[k] = lane;
-      ml.pos[k] = pos;
-    }
-    if (m2) {
-      const int k = __popcll(b1) + __popcll(b2 & below);
-      ml.phys[k] = win;
-      ml.pos[k] = lane;
-    }
     const unsigned long long z = __ballot(lane < w && s_zero[lane]);
-    if (lane == 0) ml.cnt = __popcll(b1) + __popcll(b2);
     if (g == 0) {
-      if (lane < w) a.ipiv[lane] = a.r0 + from;
+      if (lane < w) {
+        a.ipiv[lane] = a.r0 + from;
+        a.moves[lane] = win;
+        a.moves[kPanelWMax + lane] = pos;
+      }
+      if (lane == 0) {
+        a.moves[2 * kPanelWMax] = a.o;
+        a.moves[2 * kPanelWMax + 1] = w;
+      }
       if (lane == 0 && z && *a.info == 0) *a.info = (int32_t)(a.r0 + __ffsll((long long)z));
     }
   }
@@ -905,7 +1009,6 @@ __global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {
   // every row of this workgroup to its final position (the bound is hidden
   // from the compiler, which would keep the W column masks of the loads
   // alive in scalar registers until here)
-  const int cnt = ml.cnt;
   int wst = w;
   asm volatile("" : "+s"(wst));
 #pragma unroll
@@ -929,156 +1032,7 @@ __global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {
         if (c < wst) dst[c] = P[q][c];
     }
   }
-  // The same interchanges on the outer panel's other columns (left and right
-  // of this leaf), so the recursion above needs no row swaps of its own.
-  // Each workgroup takes a disjoint slice of those columns, reads the moved
-  // rows of its slice into LDS, then writes them to their final positions.
-  const int64_t nout = a.left + a.right;
-  if (cnt == 0 || nout == 0) return;
-  const int64_t per = (nout + G - 1) / G;
-  const int64_t o0 = (int64_t)g * per;
-  const int64_t o1 = o0 + per < nout ? o0 + per : nout;
-  const int64_t chunk = kSwapStage / cnt;  // columns per pass that fit the stage
-  for (int64_t c0 = o0; c0 < o1; c0 += chunk) {
-    const int64_t nc = c0 + chunk < o1 ? chunk : o1 - c0;
-    for (int64_t e = tid; e < (int64_t)cnt * nc; e += NT) {
-      const int k = (int)(e / nc);
-      const int64_t oc = c0 + e % nc;
-      const int64_t col = oc < a.left ? oc - a.left : oc - a.left + w;
-      stage[e] = a.A[(int64_t)ml.phys[k] * a.lda + col];
-    }
-    __syncthreads();
-    for (int64_t e = tid; e < (int64_t)cnt * nc; e += NT) {
-      const int k = (int)(e / nc);
-      const int64_t oc = c0 + e % nc;
-      const int64_t col = oc < a.left ? oc - a.left : oc - a.left + w;
-      a.A[(int64_t)ml.pos[k] * a.lda + col] = stage[e];
-    }
-    __syncthreads();
-  }
 }
-
-// ---------------------------------------------------------------------------
-// Row interchange plan: the net permutation of the sequential swaps
-// ipiv[s..e) (absolute rows, ipiv[i] >= i) as (dst, src) pairs.
-constexpr int kSwapMax = 512;
-
-__global__ __launch_bounds__(64) void swap_plan_kernel(const int64_t* __restrict__ ipiv, int64_t s,
-                                                       int64_t e, int64_t* __restrict__ dst,
-                                                       int64_t* __restrict__ src,
-                                                       int* __restrict__ count) {
-  __shared__ int64_t in_src[kSwapMax];
-  __shared__ int64_t out_pos[kSwapMax];
-  __shared__ int64_t out_src[kSwapMax];
-  __shared__ int64_t piv[kSwapMax];
-  __shared__ int nout;
-  const int lane = threadIdx.x;
-  const int k = (int)(e - s);
-  for (int t = lane; t < k; t += 64) {
-    in_src[t] = s + t;
-    piv[t] = ipiv[s + t];
-  }
-  if (lane == 0) nout = 0;
-  __syncthreads();
-  for (int i = 0; i < k; ++i) {
-    const int64_t p = piv[i];
-    if (p < e) {
-      if (lane == 0 && p != s + i) {
-        const int64_t tmp = in_src[i];
-        in_src[i] = in_src[p - s];
-        in_src[p - s] = tmp;
-      }
-    } else {
-      // find p among out_pos (wave-parallel)
-      int found = -1;
-      for (int base = 0; base < nout; base += 64) {
-        const int q = base + lane;
-        const bool hit = q < nout && out_pos[q] == p;
-        const unsigned long long bal = __ballot(hit);
-        if (bal) {
-          found = base + __ffsll((long long)bal) - 1;
-          break;
-        }
-      }
-      if (lane == 0) {
-        int q = found;
-        if (q < 0) {
-          q = nout++;
-          out_pos[q] = p;
-          out_src[q] = p;
-        }
-        const int64_t tmp = in_src[i];
-        in_src[i] = out_src[q];
-        out_src[q] = tmp;
-      }
-    }
-    __syncthreads();
-  }
-  if (lane == 0) {
-    int c = 0;
-    for (int t = 0; t < k; ++t)
-      if (in_src[t] != s + t) {
-        dst[c] = s + t;
-        src[c] = in_src[t];
-        ++c;
-      }
-    for (int q = 0; q < nout; ++q)
-      if (out_src[q] != out_pos[q]) {
-        dst[c] = out_pos[q];
-        src[c] = out_src[q];
-        ++c;
-      }
-    *count = c;
-  }
-}
-
-// This workgroup's share (blockIdx.x of gridDim.x) of a copy of nc
-// entries, with 16-byte accesses when both ends are 16-byte aligned.
-template <typename T>
-__device__ inline void copy_row_part(const T* __restrict__ s, T* __restrict__ d, int64_t nc) {
-  constexpr int E = 16 / sizeof(T);
-  typedef T V __attribute__((ext_vector_type(E)));
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (((reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(d)) & 15) == 0) {
-    const int64_t nv = nc / E;
-    for (int64_t v = t0; v < nv; v += stride) reinterpret_cast<V*>(d)[v] = reinterpret_cast<const V*>(s)[v];
-    for (int64_t c = nv * E + t0; c < nc; c += stride) d[c] = s[c];
-  } else {
-    for (int64_t c = t0; c < nc; c += stride) d[c] = s[c];
-  }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void swap_gather_kernel(const T* __restrict__ A, int64_t lda,
-                                                          int64_t c0, int64_t nc,
-                                                          const int64_t* __restrict__ src,
-                                                          const int* __restrict__ count,
-                                                          T* __restrict__ tmp) {
-  const int q = blockIdx.y;
-  if (q >= *count) return;
-  copy_row_part<T>(A + src[q] * lda + c0, tmp + (int64_t)q * nc, nc);
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void swap_scatter_kernel(T* __restrict__ A, int64_t lda, int64_t c0,
-                                                           int64_t nc,
-                                                           const int64_t* __restrict__ dst,
-                                                           const int* __restrict__ count,
-                                                           const T* __restrict__ tmp) {
-  const int q = blockIdx.y;
-  if (q >= *count) return;
-  copy_row_part<T>(tmp + (int64_t)q * nc, A + dst[q] * lda + c0, nc);
-}
-
-// ---------------------------------------------------------------------------
-// U12 = inv(L11) A12 as one MFMA GEMM.  inv(L11) (unit lower, W <= kNB) is
-// built by the panel recursion itself: every leaf inverts its own diagonal
-// block (trtri_diag_kernel, FP64 arithmetic rounded to T) and every split
-// of the recursion joins the inverses of its halves with two GEMMs,
-// X21 = -X22 (L21 X11).
-constexpr int kTri = 64;
-constexpr int kNB = 512;  // outer panel width of the blocked LU
 
 // Inverse of the sz x sz (sz <= 64) unit-lower block at L into X[0:sz, 0:sz]
 // (zeros above the diagonal included), in FP64 arithmetic.  Blocked by 16:
@@ -1087,10 +1041,9 @@ constexpr int kNB = 512;  // outer panel width of the blocked LU
 //   2. block rows I = 1..3 in turn: S = L[I, 0:I] X[0:I, 0:I], then
 //      X[I, 0:I] = -X_II S (two barriers per block row).
 // Rows and columns from sz to 64 are padded with the identity.
-// NT = 16 for the 16-wide leaves: the 16 x 16 substitution alone, without
-// the three empty block-row joins of the 64 x 64 case.
+// NT = 16 for leaves of at most 16 columns: the 16 x 16 substitution alone.
 template <typename T, int NT>
-__global__ __launch_bounds__(256) void trtri_diag_kernel(const T* __restrict__ L, int64_t ldl, int sz,
+__device__ __forceinline__ void unit_inverse(const T* __restrict__ L, int64_t ldl, int sz,
                                                         T* __restrict__ X, int64_t ldx) {
   __shared__ double Ls[NT * (NT - 1) / 2];  // strictly lower part, packed by rows
   __shared__ double Xs[NT][NT + 1];
@@ -1152,6 +1105,220 @@ __global__ __launch_bounds__(256) void trtri_diag_kernel(const T* __restrict__ L
   }
 }
 
+// A factored leaf's effect on the outer panel's other columns: its row
+// interchanges, and on the columns to its right U12 = inv(L11) A12 of its
+// rows.  A workgroup takes 64 columns: it reads the winners' rows (which
+// become the leaf's rows) and the rows they displace, then writes both; on
+// the right the winners' rows pass through the triangular solve first (16
+// columns per wave, MFMA tiles, the 16 x 16 diagonal blocks inverted on the
+// way).  Bound by the latency of its few dependent steps.  One launch instead of the
+// interchanges inside the leaf, the inverse of its 64 x 64 block (20 us in one
+// workgroup), a copy and one or two products per split of the panel.
+// SOLVE false (recursive panels): the interchanges alone, and in the last
+// workgroup the inverse of the leaf's diagonal block into ride.X.
+template <typename T, bool SOLVE>
+__global__ __launch_bounds__(256) void panel_apply_kernel(T* __restrict__ A, int64_t lda, int lcol, int w, int pw,
+                                                          const int* __restrict__ moves, InvArgs<T> ride) {
+  constexpr int LS = kTri + 16 / (int)sizeof(T);
+  __shared__ T Ls[SOLVE ? kTri : 1][LS], Ss[SOLVE ? kTri : 1][kTri + 1];
+  __shared__ double inv[4][16][17];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int nleft = (lcol + kTri - 1) / kTri;
+  const int nright = (pw - lcol - w + kTri - 1) / kTri;
+  if ((int)blockIdx.x >= nleft + nright) {
+    if constexpr (SOLVE) {
+      inverse_rows<T>(ride, (int)blockIdx.x - nleft - nright, inv);
+    } else if (w <= 16) {
+      unit_inverse<T, 16>(A + lcol, lda, w, ride.X, ride.ldx);
+    } else {
+      unit_inverse<T, kTri>(A + lcol, lda, w, ride.X, ride.ldx);
+    }
+    return;
+  }
+  const bool right = (int)blockIdx.x >= nleft;
+  const int c0 = right ? lcol + w + ((int)blockIdx.x - nleft) * kTri : (int)blockIdx.x * kTri;
+  const int nc = (right ? pw : lcol) - c0 < kTri ? (right ? pw : lcol) - c0 : kTri;
+  T* C = A + c0;
+  T vs[16], vd[16];
+  int win[16], pos[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    const int r = wv + 4 * t;
+    win[t] = r < w ? moves[r] : r;
+    pos[t] = r < w ? moves[kPanelWMax + r] : r;
+  }
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    const int r = wv + 4 * t;
+    vs[t] = r < w && lane < nc ? C[(int64_t)win[t] * lda + lane] : T(0);
+    vd[t] = r < w && pos[t] >= w && lane < nc ? C[(int64_t)r * lda + lane] : T(0);
+  }
+  if (SOLVE && right) {
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      const int r = wv + 4 * t;
+      Ls[r][lane] = r < w && lane < r ? A[(int64_t)r * lda + lcol + lane] : T(0);
+    }
+#pragma unroll
+    for (int t = 0; t < 16; ++t) Ss[wv + 4 * t][lane] = vs[t];
+  }
+  // every row is in registers or LDS before any is overwritten
+  __builtin_amdgcn_s_waitcnt(0xF70);
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    const int r = wv + 4 * t;
+    if (r >= w || lane >= nc) continue;
+    if (pos[t] >= w) C[(int64_t)pos[t] * lda + lane] = vd[t];
+    if (!SOLVE || !right) C[(int64_t)r * lda + lane] = vs[t];
+  }
+  if (!SOLVE || !right) return;
+  tri_inv16([&](int i, int k) -> double { return (double)Ls[16 * wv + i][16 * wv + k]; }, inv[wv]);
+  __syncthreads();
+  const int m = lane & 15;
+  typename Mma<T>::acc_t acc[4];
+#pragma unroll
+  for (int I = 0; I < 4; ++I)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[I][e] = Ss[16 * I + Mma<T>::row(lane, e)][16 * wv + m];
+  tri_solve64<T>(
+      acc, [&](int i, int k) -> T { return Ls[i][k]; }, inv);
+  if (16 * wv + m >= nc) return;
+#pragma unroll
+  for (int I = 0; I < 4; ++I)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 16 * I + Mma<T>::row(lane, e);
+      if (r < w) C[(int64_t)r * lda + 16 * wv + m] = acc[I][e];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// End of an outer panel of W columns at absolute row s, in one launch: the
+// last row block of the inverse (workgroups 0 .. v.b), and the panel's net
+// row interchange as (dst, src) pairs (the last workgroup), composed from
+// the leaves' moves in order (moves[l]: winners and final positions of the
+// first rows, relative to the leaf's first row, its column and width).  Each
+// leaf's moves are one parallel step: content[t] is the row now at position
+// t < W, and positions past the panel sit in a hash table once a winner came
+// from there.  (Replaying the 512 interchanges one by one took 50-150 us.)
+constexpr int kSwapMax = 512;
+constexpr int kPlanSlots = 2048;
+
+template <typename T>
+__global__ __launch_bounds__(256) void panel_finish_kernel(InvArgs<T> v, const int* __restrict__ moves, int nl, int W,
+                                                           int64_t s, int64_t* __restrict__ dst,
+                                                           int64_t* __restrict__ src, int* __restrict__ count) {
+  __shared__ double inv[4][16][17];
+  __shared__ int content[kSwapMax];
+  __shared__ int key[kPlanSlots], held[kPlanSlots];  // positions past the panel (-1: free), rows there
+  __shared__ int nout;
+  if ((int)blockIdx.x <= v.b) {
+    inverse_rows<T>(v, blockIdx.x, inv);
+    return;
+  }
+  const int tid = threadIdx.x;
+  for (int t = tid; t < W; t += 256) content[t] = t;
+  for (int t = tid; t < kPlanSlots; t += 256) key[t] = -1;
+  if (tid == 0) nout = 0;
+  __syncthreads();
+  auto slot_of = [&](int p, bool insert) -> int {
+    unsigned h = ((unsigned)p * 2654435761u) >> 21;
+    for (;; h = (h + 1) & (kPlanSlots - 1)) {
+      const int k = key[h];
+      if (k == p) return (int)h;
+      if (insert && k == -1) {
+        const int old = atomicCAS(&key[h], -1, p);
+        if (old == -1) {
+          held[h] = p;  // nothing moved there yet
+          return (int)h;
+        }
+        if (old == p) return (int)h;
+      }
+    }
+  };
+  for (int l = 0; l < nl; ++l, moves += kMoveStride) {
+    const int o = moves[2 * kPanelWMax], w = moves[2 * kPanelWMax + 1];
+    int top = 0, low = 0, to = -1;
+    if (tid < w) {
+      const int p = o + moves[tid];
+      top = p < W ? content[p] : held[slot_of(p, true)];
+      to = o + moves[kPanelWMax + tid];
+      low = content[o + tid];
+    }
+    __syncthreads();
+    if (tid < w) {
+      content[o + tid] = top;
+      // a displaced row goes where a winner from below the leaf came from
+      if (to >= o + w) {
+        if (to < W)
+          content[to] = low;
+        else
+          held[slot_of(to, false)] = low;
+      }
+    }
+    __syncthreads();
+  }
+  for (int t = tid; t < W; t += 256)
+    if (content[t] != t) {
+      const int k = atomicAdd(&nout, 1);
+      dst[k] = s + t;
+      src[k] = s + content[t];
+    }
+  for (int t = tid; t < kPlanSlots; t += 256)
+    if (key[t] != -1 && held[t] != key[t]) {
+      const int k = atomicAdd(&nout, 1);
+      dst[k] = s + key[t];
+      src[k] = s + held[t];
+    }
+  __syncthreads();
+  if (tid == 0) *count = nout;
+}
+
+// This workgroup's share (blockIdx.x of gridDim.x) of a copy of nc
+// entries, with 16-byte accesses when both ends are 16-byte aligned.
+template <typename T>
+__device__ inline void copy_row_part(const T* __restrict__ s, T* __restrict__ d, int64_t nc) {
+  constexpr int E = 16 / sizeof(T);
+  typedef T V __attribute__((ext_vector_type(E)));
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (((reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(d)) & 15) == 0) {
+    const int64_t nv = nc / E;
+    for (int64_t v = t0; v < nv; v += stride) reinterpret_cast<V*>(d)[v] = reinterpret_cast<const V*>(s)[v];
+    for (int64_t c = nv * E + t0; c < nc; c += stride) d[c] = s[c];
+  } else {
+    for (int64_t c = t0; c < nc; c += stride) d[c] = s[c];
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void swap_gather_kernel(const T* __restrict__ A, int64_t lda,
+                                                          int64_t c0, int64_t nc,
+                                                          const int64_t* __restrict__ src,
+                                                          const int* __restrict__ count,
+                                                          T* __restrict__ tmp) {
+  const int q = blockIdx.y;
+  if (q >= *count) return;
+  copy_row_part<T>(A + src[q] * lda + c0, tmp + (int64_t)q * nc, nc);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void swap_scatter_kernel(T* __restrict__ A, int64_t lda, int64_t c0,
+                                                           int64_t nc,
+                                                           const int64_t* __restrict__ dst,
+                                                           const int* __restrict__ count,
+                                                           const T* __restrict__ tmp) {
+  const int q = blockIdx.y;
+  if (q >= *count) return;
+  copy_row_part<T>(tmp + (int64_t)q * nc, A + dst[q] * lda + c0, nc);
+}
+
+// ---------------------------------------------------------------------------
+// U12 = inv(L11) A12 as one MFMA GEMM.  inv(L11) (unit lower, W <= kNB) is
+// built with the panel, a row block per leaf.
+constexpr int kNB = 512;  // outer panel width of the blocked LU
+
 // dst (rows x cols, ld ldd) = src (ld lds)
 template <typename T>
 __global__ __launch_bounds__(256) void copy_block_kernel(const T* __restrict__ src, int64_t lds, int rows,
@@ -1201,10 +1368,11 @@ struct LuCtx {
   unsigned seq;     // steps taken by the panel launches so far
   LuScratch<T> sc;
   int G_max;
-  int wleaf = kPanelWMax;  // leaf width of the recursion
-  int64_t pc0 = 0;  // outer panel being factored: columns [pc0, pc0 + pw)
-  int pw = 0;
-  bool on_panel_stream = false;  // the panel stream's context (runs beside the trailing update)
+  int wleaf = kPanelWMax;  // widest leaf
+  bool recursive = false;  // panels by recursive halving (kRecursiveRows)
+  T* panel_tmp = nullptr;  // [kNB][kNB] staging of the recursion
+  int* moves = nullptr;  // [kMaxLeaves][kMoveStride] of the panel being factored
+  int nleaves = 0;       // leaves factored so far in that panel (recursive panels)
 };
 
 // Upper bound on the workgroups of one leaf launch (0: the CU count).
@@ -1236,7 +1404,7 @@ static bool lone_leaf(int64_t m, int w, int& nt, LeafShape& shape) {
 }
 
 template <typename T>
-static int leaf(LuCtx<T>& c, int64_t r0, int w) {
+static int leaf(LuCtx<T>& c, int64_t r0, int o, int w, int* moves, const InvArgs<T>& inv) {
   const DeviceInfo& di = device_info();
   const int64_t m = c.n - r0;
   int cap = g_panel_groups.load(std::memory_order_relaxed);
@@ -1269,9 +1437,10 @@ static int leaf(LuCtx<T>& c, int64_t r0, int w) {
   a.w = w;
   a.R = R;
   a.r0 = r0;
-  a.left = r0 - c.pc0;
-  a.right = c.pc0 + c.pw - (r0 + w);
-  RBFX_REQUIRE(a.left >= 0 && a.right >= 0, "leaf outside its outer panel");
+  a.G = G;
+  a.moves = moves;
+  a.o = o;
+  a.inv = inv;
   RBFX_REQUIRE(w >= 1 && w <= kPanelWMax, "leaf width %d out of range", w);
   a.ipiv = c.ipiv + r0;
   a.cand = c.cand;
@@ -1291,7 +1460,7 @@ static int leaf(LuCtx<T>& c, int64_t r0, int w) {
   // the same but goes through a separate device queue, which added ~60 us
   // of dispatch latency per leaf, measured.)
 #define RBFX_LEAF(ROWS_, W_, NT_) \
-  hipLaunchKernelGGL((panel_kernel<T, ROWS_, W_, NT_>), dim3(G), dim3(NT_), 0, c.s, a)
+  hipLaunchKernelGGL((panel_kernel<T, ROWS_, W_, NT_>), dim3(G + inv.b + 1), dim3(NT_), 0, c.s, a)
   if (nt != kPanelThreads) {
     if (nt == 512 && rows == 1) RBFX_LEAF(1, kPanelWMax, 512);
     else if (nt == 768 && rows == 1 && sizeof(T) == 8) RBFX_LEAF(1, kPanelWMax, sizeof(T) == 8 ? 768 : 512);
@@ -1316,42 +1485,11 @@ static int leaf(LuCtx<T>& c, int64_t r0, int w) {
   return RBFX_OK;
 }
 
-// Net row-interchange plan of the swaps ipiv[s..e) into dst's plan buffers,
-// enqueued on c's stream.
-template <typename T>
-static int make_plan(LuCtx<T>& c, LuScratch<T>& dst, int64_t s, int64_t e) {
-  RBFX_REQUIRE(e - s <= kSwapMax, "too many swaps in one plan");
-  hipLaunchKernelGGL(swap_plan_kernel, dim3(1), dim3(64), 0, c.s, c.ipiv, s, e, dst.plan_dst, dst.plan_src,
-                     dst.plan_count);
-  RBFX_CHECK_LAUNCH();
-  dst.plan_s = s;
-  dst.plan_e = e;
-  return RBFX_OK;
-}
-
-// Inverse of a leaf's w x w unit-lower diagonal block (at (r0, r0)) into X,
-// enqueued on c's stream.
-template <typename T>
-static int leaf_inverse(LuCtx<T>& c, int64_t r0, int w, T* X, int64_t ldx) {
-  RBFX_REQUIRE(w <= kTri, "leaf wider than the diagonal inverse kernel");
-  const int pid = prof_start(sizeof(T) == 8 ? "trtri_f64" : "trtri_f32", c.s);
-  if (w <= 16)
-    hipLaunchKernelGGL((trtri_diag_kernel<T, 16>), dim3(1), dim3(256), 0, c.s, c.A + r0 * c.lda + r0, c.lda, w,
-                       X, ldx);
-  else
-    hipLaunchKernelGGL((trtri_diag_kernel<T, kTri>), dim3(1), dim3(256), 0, c.s, c.A + r0 * c.lda + r0, c.lda, w,
-                       X, ldx);
-  RBFX_CHECK_LAUNCH();
-  prof_stop(pid, c.s, (double)w * w * w / 3.0, (double)sizeof(T) * w * w);
-  return RBFX_OK;
-}
-
 // Apply the swaps ipiv[s..e) to columns [c0, c0+nc).
 template <typename T>
 static int apply_swaps(LuCtx<T>& c, int64_t s, int64_t e, int64_t c0, int64_t nc) {
   if (nc <= 0 || e <= s) return RBFX_OK;
-  int st;
-  if ((c.sc.plan_s != s || c.sc.plan_e != e) && (st = make_plan(c, c.sc, s, e))) return st;
+  RBFX_REQUIRE(c.sc.plan_s == s && c.sc.plan_e == e, "no plan of these interchanges");
   const int maxcnt = (int)(2 * (e - s));
   const int pid = prof_start("row_swaps", c.s);
   // process the columns in slices that fit the staging buffer
@@ -1371,66 +1509,146 @@ static int apply_swaps(LuCtx<T>& c, int64_t s, int64_t e, int64_t c0, int64_t nc
   return RBFX_OK;
 }
 
+// Leading dimension of staged blocks: rows that the LDS-DMA product can read.
+constexpr int64_t kStageAlign = 16;
+
 // U12 = X A12 with X = inv(L11) of the W x W diagonal block at r0 (ld ldx)
 // and columns [col, col+ncols): staged copy of A12, then one GEMM.
 template <typename T>
-static int trsm(LuCtx<T>& c, int64_t r0, int W, const T* X, int64_t ldx, int64_t col, int64_t ncols) {
+static int trsm(LuCtx<T>& c, int64_t r0, int W, const T* X, int64_t ldx, int64_t col, int64_t ncols, T* tmp,
+                int64_t tmp_elems, bool on_panel_stream = false) {
   if (ncols <= 0) return RBFX_OK;
   int st;
   const int pid = prof_start(sizeof(T) == 8 ? "trsm_f64" : "trsm_f32", c.s);
   T* B = c.A + r0 * c.lda + col;
-  const int64_t slice = std::max<int64_t>((int64_t)GBN, c.sc.swap_tmp_elems / W);
+  const int64_t slice = std::max<int64_t>((int64_t)GBN, tmp_elems / W / kStageAlign * kStageAlign);
   for (int64_t off = 0; off < ncols; off += slice) {
     const int64_t w = std::min<int64_t>(slice, ncols - off);
+    const int64_t ldt = ceil_div(w, kStageAlign) * kStageAlign;
     hipLaunchKernelGGL((copy_block_kernel<T>), dim3((unsigned)std::min<int64_t>(ceil_div(w, 256), 64), W),
-                       dim3(256), 0, c.s, B + off, c.lda, W, w, c.sc.swap_tmp, w);
+                       dim3(256), 0, c.s, B + off, c.lda, W, w, tmp, ldt);
     RBFX_CHECK_LAUNCH();
-    if ((st = gemm_launch<T, 1>(W, w, W, T(1), X, ldx, c.sc.swap_tmp, w, T(0), B + off, c.lda, c.s,
-                                c.on_panel_stream)))
+    if ((st = gemm_launch<T, 1>(W, w, W, T(1), X, ldx, tmp, ldt, T(0), B + off, c.lda, c.s,
+                                on_panel_stream && sizeof(T) == 4, !c.recursive)))
       return st;
   }
   prof_stop(pid, c.s, 2.0 * W * W * ncols, 3.0 * sizeof(T) * W * ncols);
   return RBFX_OK;
 }
 
-// Recursive factorisation of the panel rows [r0, n) x columns [r0, r0+W).
-// It also leaves X = inv(L11) of the panel's W x W unit-lower diagonal block
-// (ld ldx) in X's lower triangle; X's strictly upper part must hold zeros
-// (the buffer is cleared once per factorisation and only ever receives
-// lower-triangular entries).
+// Factorisation of the panel rows [r0, n) x columns [r0, r0+W), leaf by leaf:
+// each leaf's interchanges and triangular solve on the panel's other columns
+// in one launch, then the rank-w update of the columns to its right.  It also
+// leaves X = inv(L11) of the W x W unit-lower diagonal block (ld ldx) in X's
+// lower triangle, 64 rows riding along with the leaf after them and the last
+// ones with the interchange plan in out's plan buffers; X's strictly upper
+// part must hold zeros (the buffer is cleared once per factorisation and
+// only ever receives lower-triangular entries).
 template <typename T>
-static int panel(LuCtx<T>& c, int64_t r0, int W, T* X, int64_t ldx) {
+static int panel(LuCtx<T>& c, int64_t r0, int W, T* X, int64_t ldx, LuScratch<T>& out) {
+  int st;
+  RBFX_REQUIRE(W <= kSwapMax && kTri % c.wleaf == 0, "panel too wide");
+  InvArgs<T> inv;
+  inv.P = c.A + r0 * c.lda + r0;
+  inv.lda = c.lda;
+  inv.X = X;
+  inv.ldx = ldx;
+  int nl = (W + c.wleaf - 1) / c.wleaf;
+  if (c.recursive) {
+    c.nleaves = 0;
+    if ((st = panel_recursive(c, r0, W, r0, W, X, ldx))) return st;
+    nl = c.nleaves;
+  }
+  for (int o = 0, l = 0; !c.recursive && o < W; o += c.wleaf, ++l) {
+    const int w = std::min(c.wleaf, W - o);
+    const int rest = W - o - w;
+    int* moves = c.moves + (size_t)l * kMoveStride;
+    const bool whole = o > 0 && o % kTri == 0;  // the leaf before ended a row block
+    inv.b = whole ? o / kTri - 1 : -1;
+    inv.w = kTri;
+    // (narrow leaves keep their registers low and leave the inverse to the
+    // launch after them)
+    InvArgs<T> ride = inv, none = inv;
+    none.b = -1;
+    if ((st = leaf(c, r0 + o, o, w, moves, w > kPanelWNarrow ? inv : none))) return st;
+    if (w > kPanelWNarrow) ride.b = -1;
+    if (o > 0 || rest > 0) {
+      const int pid = prof_start(sizeof(T) == 8 ? "panel_apply_f64" : "panel_apply_f32", c.s);
+      hipLaunchKernelGGL((panel_apply_kernel<T, true>), dim3((unsigned)(ceil_div(o, kTri) + ceil_div(rest, kTri) + ride.b + 1)),
+                         dim3(256), 0, c.s, c.A + (r0 + o) * c.lda + r0, c.lda, o, w, W, (const int*)moves, ride);
+      RBFX_CHECK_LAUNCH();
+      prof_stop(pid, c.s, (double)w * w * rest, 4.0 * sizeof(T) * w * (W - w));
+    }
+    T* R = c.A + (r0 + o) * c.lda + r0 + o + w;  // the leaf's rows, columns to its right
+    if ((st = gemm<T>(c.n - r0 - o - w, rest, w, T(-1), R + (int64_t)w * c.lda - w, c.lda, R, c.lda, T(1),
+                      R + (int64_t)w * c.lda, c.lda, c.s, true)))
+      return st;
+  }
+  inv.b = c.recursive ? -1 : (W - 1) / kTri;
+  inv.w = W - kTri * inv.b;
+  hipLaunchKernelGGL((panel_finish_kernel<T>), dim3(inv.b + 2), dim3(256), 0, c.s, inv, (const int*)c.moves, nl, W,
+                     r0, out.plan_dst, out.plan_src, out.plan_count);
+  RBFX_CHECK_LAUNCH();
+  out.plan_s = r0;
+  out.plan_e = r0 + W;
+  return RBFX_OK;
+}
+
+// FP64 systems of at most this many rows take the recursive panels: U12 by
+// the inverse of the half panel's whole diagonal block, as opposed to block
+// substitution.  Both are backward stable (same ||P A - L U||), but implicit
+// time stepping at these sizes goes through tens of solves with kappa(K) ~
+// 1e10, where another rounding of the factors moves its results by up to 2e-9
+// (60 x 60 nodes, 8 steps); larger systems and the FP32 factors (which only
+// precondition) take the leaf-by-leaf panels, which are faster: FP64 LU at
+// n = 10,006 47.0 against 60.1 ms.
+constexpr int64_t kRecursiveRows = 4096;
+constexpr int kMaxLeaves = kNB / 8;  // the recursion splits no narrower than 8
+
+// Recursive factorisation of the panel columns [r0, r0+W) of the outer panel
+// that starts at column pc0 and is pw wide, X = inv(L11) as below; each half's
+// inverse is joined with X21 = -X22 (L21 X11).
+template <typename T>
+static int panel_recursive(LuCtx<T>& c, int64_t pc0, int pw, int64_t r0, int W, T* X, int64_t ldx) {
   int st;
   if (W <= c.wleaf) {
-    if ((st = leaf(c, r0, W))) return st;
-    return leaf_inverse(c, r0, W, X, ldx);
+    const int o = (int)(r0 - pc0);
+    int* moves = c.moves + (size_t)c.nleaves++ * kMoveStride;
+    RBFX_REQUIRE(c.nleaves <= kMaxLeaves, "too many leaves in a panel");
+    InvArgs<T> v;
+    if ((st = leaf(c, r0, o, W, moves, v))) return st;
+    v.X = X;
+    v.ldx = ldx;
+    const int pid = prof_start(sizeof(T) == 8 ? "panel_apply_f64" : "panel_apply_f32", c.s);
+    hipLaunchKernelGGL((panel_apply_kernel<T, false>),
+                       dim3((unsigned)(ceil_div(o, kTri) + ceil_div(pw - o - W, kTri) + 1)), dim3(256), 0, c.s,
+                       c.A + r0 * c.lda + pc0, c.lda, o, W, pw, (const int*)moves, v);
+    RBFX_CHECK_LAUNCH();
+    prof_stop(pid, c.s, (double)W * W * W / 3.0, 4.0 * sizeof(T) * W * (pw - W));
+    return RBFX_OK;
   }
   const int W1 = std::max(8, (W / 2 + 7) / 8 * 8);
   const int W2 = W - W1;
-  // (every leaf applies its row interchanges to all columns of the outer
-  // panel itself, so the halves need no swaps here)
-  if ((st = panel(c, r0, W1, X, ldx))) return st;
-  if ((st = trsm(c, r0, W1, X, ldx, r0 + W1, W2))) return st;
+  if ((st = panel_recursive(c, pc0, pw, r0, W1, X, ldx))) return st;
+  if ((st = trsm(c, r0, W1, X, ldx, r0 + W1, W2, c.panel_tmp, (int64_t)kNB * kNB, true))) return st;
   const int64_t m2 = c.n - r0 - W1;
   const T* L21 = c.A + (r0 + W1) * c.lda + r0;
   if ((st = gemm<T>(m2, W2, W1, T(-1), L21, c.lda, c.A + r0 * c.lda + r0 + W1, c.lda, T(1),
-                    c.A + (r0 + W1) * c.lda + r0 + W1, c.lda, c.s, true)))
+                    c.A + (r0 + W1) * c.lda + r0 + W1, c.lda, c.s, true, false)))
     return st;
   T* X22 = X + (int64_t)W1 * ldx + W1;
-  if ((st = panel(c, r0 + W1, W2, X22, ldx))) return st;
+  if ((st = panel_recursive(c, pc0, pw, r0 + W1, W2, X22, ldx))) return st;
   // L21 (rows r0+W1 .. r0+W) is final now: later pivots only move rows
-  // >= r0+W.  X21 = -X22 (L21 X11), the product staged in the panel's
-  // swap buffer.
-  RBFX_REQUIRE((int64_t)W1 * W2 <= c.sc.swap_tmp_elems, "inverse staging too small");
-  T* Tm = c.sc.swap_tmp;
+  // >= r0+W
   const int pid = prof_start(sizeof(T) == 8 ? "trtri_f64" : "trtri_f32", c.s);
-  if ((st = gemm_launch<T, 2>(W2, W1, W1, T(1), L21, c.lda, X, ldx, T(0), Tm, W1, c.s, c.on_panel_stream)))
+  if ((st = gemm_launch<T, 2>(W2, W1, W1, T(1), L21, c.lda, X, ldx, T(0), c.panel_tmp, W1, c.s, true, false)))
     return st;
-  st = gemm_launch<T, 2>(W2, W1, W2, T(-1), X22, ldx, Tm, W1, T(0), X + (int64_t)W1 * ldx, ldx, c.s,
-                         c.on_panel_stream);
+  st = gemm_launch<T, 2>(W2, W1, W2, T(-1), X22, ldx, c.panel_tmp, W1, T(0), X + (int64_t)W1 * ldx, ldx, c.s, true,
+                         false);
   prof_stop(pid, c.s, 2.0 * W2 * W1 * (double)(W1 + W2), (double)sizeof(T) * 3.0 * W1 * W2);
   return st;
 }
+
 
 static size_t getrf_ws_bytes(int64_t n, int bytes) {
   const int G = 1024;  // upper bound on workgroups of a leaf
@@ -1438,16 +1656,16 @@ static size_t getrf_ws_bytes(int64_t n, int bytes) {
   b += ws_round((size_t)2 * G * kRecWords * 8);   // cand records
   b += ws_round((size_t)2 * kKeyMaxGroups * (kPanelWMax + 2) * 2 * bytes);  // cand_row (tagged)
   b += ws_round(64);                              // status
-  for (int q = 0; q < 3; ++q) {                   // two slots of the main stream, one of the panel stream
+  for (int q = 0; q < 2; ++q) {                   // two slots, filled by the panel stream in turn
     b += ws_round((size_t)2 * kSwapMax * 8) * 2;  // plan dst / src
     b += ws_round(64);                            // plan count
     b += ws_round((size_t)kNB * kNB * bytes);     // inverse of the diagonal block
   }
   // main stream: staging of row swaps (2*NB rows x min(n, 8192) columns) and
   // of the triangular solve's right-hand side (NB x n)
-  b += ws_round((size_t)std::max<int64_t>(2 * kNB * std::min<int64_t>(n, 8192), (int64_t)kNB * n) * bytes);
-  // panel stream: swaps and solves inside one panel (at most 2*NB x NB)
-  b += ws_round((size_t)2 * kNB * kNB * bytes);
+  b += ws_round((size_t)std::max<int64_t>(2 * kNB * std::min<int64_t>(n, 8192), (int64_t)kNB * ceil_div(n, kStageAlign) * kStageAlign) * bytes);
+  b += ws_round((size_t)kMaxLeaves * kMoveStride * 4);  // moves of one panel's leaves
+  b += ws_round((size_t)kNB * kNB * bytes);             // staging of the recursive panels
   return b;
 }
 
@@ -1535,11 +1753,15 @@ static int getrf(int64_t n, T* A, int64_t lda, int64_t* ipiv, void* work, size_t
   unsigned* ctl = ws.take<unsigned>(16);
   c.status = reinterpret_cast<int*>(ctl + 1);
   // main stream: two slots of (plan, inverse) filled by the panel stream
-  // for alternate steps, one staging buffer; panel stream: its own scratch
-  LuScratch<T> slot[2], sc_panel;
-  const int64_t tmp_main = std::max<int64_t>(2 * kNB * std::min<int64_t>(n, 8192), (int64_t)kNB * n);
-  const bool ok = carve_scratch(ws, slot[0], tmp_main) && carve_scratch(ws, slot[1], 0) &&
-                  carve_scratch(ws, sc_panel, (int64_t)2 * kNB * kNB);
+  // for alternate steps, one staging buffer
+  LuScratch<T> slot[2];
+  const int64_t tmp_main =
+      std::max<int64_t>(2 * kNB * std::min<int64_t>(n, 8192), (int64_t)kNB * ceil_div(n, kStageAlign) * kStageAlign);
+  bool ok = carve_scratch(ws, slot[0], tmp_main) && carve_scratch(ws, slot[1], 0);
+  c.moves = ws.take<int>((size_t)kMaxLeaves * kMoveStride);
+  c.panel_tmp = ws.take<T>((size_t)kNB * kNB);
+  c.recursive = sizeof(T) == 8 && n <= kRecursiveRows;
+  ok = ok && c.moves && c.panel_tmp;
   slot[1].swap_tmp = slot[0].swap_tmp;
   slot[1].swap_tmp_elems = slot[0].swap_tmp_elems;
   RBFX_REQUIRE(ok && c.cand && c.cand_row, "workspace carve failed");
@@ -1567,25 +1789,20 @@ static int getrf(int64_t n, T* A, int64_t lda, int64_t* ipiv, void* work, size_t
   // panel context: same matrix and pivot records, own stream and scratch
   LuCtx<T> cp = c;
   cp.s = ps->s;
-  cp.on_panel_stream = true;
-  cp.sc = sc_panel;
   hipEvent_t ready = ps->ev[0], done = ps->ev[1];
   // Panel stream, per step: factor the panel (which also leaves the inverse
   // of its diagonal block in the main stream's slot), then the
   // row-interchange plan for that slot.
-  // Narrow leaves only for panels that run beside a trailing update (not
-  // for panel 0, which runs alone).
+  // Narrow leaves only on request, and only for panels that run beside a
+  // trailing update (not for panel 0, which runs alone).
   auto panel_step = [&](int64_t r0, int W, LuScratch<T>& out, bool beside_update) -> int {
     int e;
     const int pid = prof_start(sizeof(T) == 8 ? "panel_step_f64" : "panel_step_f32", cp.s);
-    cp.pc0 = r0;
-    cp.pw = W;
     const int64_t nl = g_narrow_leaf_rows.load(std::memory_order_relaxed);
-    const int64_t narrow_rows = nl != 0 ? nl : sizeof(T) == 8 ? kNarrowLeafRows : -1;
-    cp.wleaf = beside_update && narrow_rows > 0 && n - r0 >= narrow_rows ? kPanelWNarrow : kPanelWMax;
-    if ((e = panel(cp, r0, W, out.tri_inv, (int64_t)kNB))) return e;
+    cp.wleaf = beside_update && nl > 0 && n - r0 >= nl ? kPanelWNarrow : kPanelWMax;
+    if ((e = panel(cp, r0, W, out.tri_inv, (int64_t)kNB, out))) return e;
     prof_stop(pid, cp.s, (double)(n - r0) * W * W, 0.0);
-    return make_plan(cp, out, r0, r0 + W);
+    return RBFX_OK;
   };
   // panel 0 after everything queued so far on the caller's stream
   RBFX_HIP(hipEventRecord(ready, s));
@@ -1616,14 +1833,16 @@ static int getrf(int64_t n, T* A, int64_t lda, int64_t* ipiv, void* work, size_t
     // waits for the host to reach the long update.
     const int Wn = (int)std::min<int64_t>(kNB, rest);
     if ((st = apply_swaps(c, k0, k1, k1, Wn))) return st;
-    if ((st = trsm(c, k0, W, c.sc.tri_inv, (int64_t)kNB, k1, Wn))) return st;
-    if ((st = gemm<T>(rest, Wn, W, T(-1), L21, lda, U12, lda, T(1), A22, lda, s))) return st;
+    if ((st = trsm(c, k0, W, c.sc.tri_inv, (int64_t)kNB, k1, Wn, c.sc.swap_tmp, c.sc.swap_tmp_elems))) return st;
+    if ((st = gemm<T>(rest, Wn, W, T(-1), L21, lda, U12, lda, T(1), A22, lda, s, false, !c.recursive))) return st;
     RBFX_HIP(hipEventRecord(ready, s));
     if ((st = apply_swaps(c, k0, k1, 0, k0))) return st;
     if (rest > Wn) {
       if ((st = apply_swaps(c, k0, k1, k1 + Wn, rest - Wn))) return st;
-      if ((st = trsm(c, k0, W, c.sc.tri_inv, (int64_t)kNB, k1 + Wn, rest - Wn))) return st;
-      if ((st = gemm<T>(rest, rest - Wn, W, T(-1), L21, lda, U12 + Wn, lda, T(1), A22 + Wn, lda, s)))
+      if ((st = trsm(c, k0, W, c.sc.tri_inv, (int64_t)kNB, k1 + Wn, rest - Wn, c.sc.swap_tmp,
+                     c.sc.swap_tmp_elems))) return st;
+      if ((st = gemm<T>(rest, rest - Wn, W, T(-1), L21, lda, U12 + Wn, lda, T(1), A22 + Wn, lda, s, false,
+                        !c.recursive)))
         return st;
     }
     RBFX_HIP(hipStreamWaitEvent(cp.s, ready, 0));
