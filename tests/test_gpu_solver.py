@@ -131,6 +131,39 @@ def test_eval_value_gradient_laplacian():
         assert np.abs(l - ref[R.LAP]).max() <= 1e-12 * max(sc[R.LAP], 1)
 
 
+@pytest.mark.parametrize("kind,param", C.KINDS)
+@pytest.mark.parametrize("N,P", [(5, 1), (17, 3), (2049, 5), (40, 2049), (33, 4096), (33, 4097), (2050, 4099)])
+def test_eval_and_transpose_every_operator(kind, param, N, P):
+    """rbfx_eval and rbfx_eval_t, one operator at a time and several at once,
+    against the oracle's closed forms: one or four points per workgroup, the
+    transpose by quarters (up to 4,096 points) and by workgroup sums, points
+    on centres, and a NaN point that stays in its own result."""
+    from updes_amd import engine as E
+    rng = np.random.default_rng(N + P)
+    ctr, pts = rng.uniform(0, 1, (N, 2)), rng.uniform(0, 1, (P, 2))
+    pts[0] = ctr[-1]
+    M = 6
+    c, w = rng.standard_normal(N + M), rng.standard_normal(P)
+    ops = R.rbf_ops(kind, param, pts[:, :1], pts[:, 1:], ctr[None, :, 0], ctr[None, :, 1])
+    mon = np.stack([R.monomial_ops(m, pts[:, 0], pts[:, 1]) for m in range(M)], axis=-1)
+    full = np.concatenate([ops, mon], axis=2)                      # (7, P, N + M)
+    ref, ref_t = full @ c, np.einsum("tpn,p->tn", full, w)
+    # |sum - exact| <= count eps sum |terms|, with the closed forms' own few eps
+    tol = 16 * np.finfo(float).eps * np.sqrt(N + P) * (np.abs(full) @ np.abs(c)).max(axis=1)
+    tol_t = 16 * np.finfo(float).eps * np.sqrt(N + P) * np.einsum("tpn,p->tn", np.abs(full), np.abs(w)).max(axis=1)
+    dctr, dpts, dc, dw = (torch.as_tensor(v).cuda() for v in (ctr, pts, c, w))
+    both = E.eval_ops(kind, param, dctr, dc, dpts, 0x7f).cpu().numpy()
+    bad = dpts.clone()
+    bad[P // 2, 1] = float("nan")
+    for t in range(7):
+        got = E.eval_ops(kind, param, dctr, dc, dpts, 1 << t)[t].cpu().numpy()
+        assert np.abs(got - ref[t]).max() <= tol[t] and np.abs(both[t] - ref[t]).max() <= tol[t]
+        got_t = E.eval_t(kind, param, dctr, M, dpts, t, dw).cpu().numpy()
+        assert np.abs(got_t - ref_t[t]).max() <= tol_t[t]
+        nan = torch.isnan(E.eval_ops(kind, param, dctr, dc, bad, 1 << t)[t]).cpu().numpy()
+        assert nan[P // 2] and nan.sum() == 1
+
+
 def test_integrate_field_matches_oracle_and_reference_test():
     """updes/tests/test_integrals.py on the GPU path: r^11, degree 3, 12 x 12,
     x^2/(1+y^2): same integral as the oracle, and |I - pi/12| < 0.1."""

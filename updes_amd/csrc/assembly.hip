@@ -292,21 +292,6 @@ constexpr int kAsmPairs = 1;
 constexpr int kAsmCols = 2 * kAsmThreads * kAsmPairs;  // columns per block
 constexpr int kAsmRows = 16;                            // rows per block
 
-// sqrt of x for 2^-900 <= x <= 2^900: the library's FP64 square-root
-// sequence (rsq estimate, a Goldschmidt step, two Newton corrections)
-// without its range scaling and its 0 / inf fixups, so the same result.
-__device__ inline double sqrt_mid(double x) {
-  const double g = __builtin_amdgcn_rsq(x);
-  double s = x * g, h = 0.5 * g;
-  const double r = __builtin_fma(-h, s, 0.5);
-  s = __builtin_fma(s, r, s);
-  h = __builtin_fma(h, r, h);
-  double d = __builtin_fma(-s, s, x);
-  s = __builtin_fma(d, h, s);
-  d = __builtin_fma(-s, s, x);
-  return __builtin_fma(d, h, s);
-}
-
 // Entry of an interior collocation row (the operator applied to
 // phi(., x_j) at x_i) without branches: apply_op's arithmetic, r = 0 and
 // the zero diagonal (j == i) as selects.  mid: every r^2 of the wave is in

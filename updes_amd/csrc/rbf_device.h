@@ -160,6 +160,21 @@ __device__ inline void radial(const Kern& k, double r, double& phi, double& f1, 
 // Squared distance, the same bits in every kernel.
 __device__ inline double dist2(double dx, double dy) { return __builtin_fma(dx, dx, dy * dy); }
 
+// sqrt of x for 2^-900 <= x <= 2^900: the library's FP64 square-root
+// sequence (rsq estimate, a Goldschmidt step, two Newton corrections)
+// without its range scaling and its 0 / inf fixups, so the same result.
+__device__ inline double sqrt_mid(double x) {
+  const double g = __builtin_amdgcn_rsq(x);
+  double s = x * g, h = 0.5 * g;
+  const double r = __builtin_fma(-h, s, 0.5);
+  s = __builtin_fma(s, r, s);
+  h = __builtin_fma(h, r, h);
+  double d = __builtin_fma(-s, s, x);
+  s = __builtin_fma(d, h, s);
+  d = __builtin_fma(-s, s, x);
+  return __builtin_fma(d, h, s);
+}
+
 __device__ inline double radial_value(const Kern& k, double r) {
   if (r == 0.0) return k.phi0;
   switch (k.kind) {
