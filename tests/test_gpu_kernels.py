@@ -167,6 +167,36 @@ def test_getrf_getrs(dtype, n):
         assert np.abs(res).max() < bound + 1e-12, (trans, np.abs(res).max(), bound)
 
 
+@pytest.mark.parametrize("n", [65, 511, 513, 700, 1100, 1536])
+def test_getrs_substitutes_in_ill_conditioned_blocks(n):
+    """FP64 diagonal blocks whose condition estimate exceeds 1e7 are solved by
+    substitution over their 64-row sub-blocks: here every block that holds one
+    of the columns (one per 200) scaled by 1e-9 (the solution is compared in
+    the unscaled unknowns).  Same result as SciPy's substitution with the same factors."""
+    import scipy.linalg as sl
+    from updes_amd import engine as E
+    _lib()
+    scale = np.ones(n)
+    scale[::200] = 1e-9
+    a = (_random_well(n, 5 * n) + 2.0 * np.sqrt(n) * np.eye(n)) * scale[None, :]
+    m = torch.zeros((n, E._ld(n)), dtype=torch.float64)
+    m[:, :n] = torch.as_tensor(a)
+    lu = E.LU(m.cuda(), n)
+    n64, n512 = -(-n // 64), -(-n // 512)
+    cond = lu.dinv.cpu().numpy()[n64 * 2 * 64 ** 2 + n512 * 2 * 512 ** 2:][:2 * n512].reshape(n512, 2)
+    assert cond[0, 1] > 1e7
+    LU, piv = lu.a[:, :n].cpu().numpy(), lu.ipiv.cpu().numpy()
+    b = np.random.default_rng(n).standard_normal(n)
+    for trans in (False, True):
+        rhs = b * scale if trans else b
+        x = lu.solve(torch.as_tensor(rhs).cuda(), trans=trans).cpu().numpy()
+        ref = sl.lu_solve((LU, piv), rhs, trans=1 if trans else 0)
+        if not trans:
+            x, ref = x * scale, ref * scale
+        rel = np.linalg.norm(x - ref) / np.linalg.norm(ref)
+        assert rel < 1e-11, (trans, rel)
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("n", [1, 63, 65, 511, 513, 1100])
 def test_getrs_prepare_inverts_diagonal_blocks(dtype, n):

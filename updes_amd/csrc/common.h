@@ -110,6 +110,41 @@ __device__ inline T ld_coh(const T* p) {
 }  // namespace rbfx
 
 namespace rbfx {
+// Sum of a double over the wave, in every lane: v += v[lane ^ off] for off =
+// 32, 16, 8, 4, 2, 1 (the order of a shuffle butterfly) without LDS traffic:
+// the two halves' and rows' values by lane swaps, then rotations and
+// permutations inside rows of 16 (after step 8 a row has period 8, so its
+// rotation by 4 is lane ^ 4).
+template <int CTRL>
+__device__ inline double dpp_f64(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+__device__ inline double wave_sum(double v) {
+  auto halves = [](double x, bool by32) -> double {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+    const auto l = by32 ? __builtin_amdgcn_permlane32_swap(lo, lo, false, false)
+                        : __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = by32 ? __builtin_amdgcn_permlane32_swap(hi, hi, false, false)
+                        : __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    const double p = __longlong_as_double((long long)(((unsigned long long)h[0] << 32) | l[0]));
+    const double q = __longlong_as_double((long long)(((unsigned long long)h[1] << 32) | l[1]));
+    return p + q;
+  };
+  v = halves(v, true);
+  v = halves(v, false);
+  v += dpp_f64<0x128>(v);  // row_ror:8
+  v += dpp_f64<0x124>(v);  // row_ror:4
+  v += dpp_f64<0x4e>(v);   // quad_perm [2,3,0,1]
+  v += dpp_f64<0xb1>(v);   // quad_perm [1,0,3,2]
+  return v;
+}
+}  // namespace rbfx
+
+namespace rbfx {
 // Optional per-launch timing with HIP events on the launch stream
 // (rbfx_profile_begin / rbfx_profile_end).  When disabled, prof_start()
 // returns -1 and prof_stop() does nothing.

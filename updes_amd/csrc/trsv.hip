@@ -117,10 +117,16 @@ __global__ void scatter_perm_kernel(const double* __restrict__ y, const int64_t*
 // workgroups of CH rows:
 //   1. fold the tiles of the superblocks already solved, in solve order
 //      (each superblock counts its solved chunks), into private partial sums;
-//   2. publish the chunk's CH accumulated values b - sum, count them in;
+//   2. publish the chunk's CH accumulated values b - sum;
 //   3. once all NCH chunks of the superblock are in, apply rows of its
 //      diagonal inverse to the superblock's SB values and publish the CH
 //      solution entries.
+// Every published value carries its own tag (two 64-bit words, each half of
+// the value beside a tag that the reset before the sweep cleared), so an
+// exchange is one trip, store to poll: the reader polls the values it needs,
+// one per thread, with no counter, and the writer does not wait for its stores.
+// The loads of the next product start between the values' departure and the
+// wait for the others'.
 // Tickets are taken in start order and each superblock has NCH consecutive
 // tickets, so the peers a workgroup waits for in step 3 have all started
 // before any workgroup of a later superblock: the waits always end.
@@ -326,12 +332,13 @@ __global__ void sbcond_kernel(int64_t nblk, const double* __restrict__ part, dou
 }
 
 // ctl[0] ticket, ctl[1] superblocks solved, ctl[2] status of the solve; the
-// s-th processed superblock owns the 128-byte line ctl[kCtlLine (s + 1) ..]:
-// word e < 3 counts its chunks that have published stage e (0: accumulated
-// values, 1: first solution, 2: its residual), word 3 its solved chunks.
-// Separate lines keep the polls of one superblock's counters off the others'.
-// Superblocks complete in order (each folds its predecessor), so ctl[1] >= k
-// means superblocks 0 .. k-1 are solved.
+// s-th processed superblock counts its solved chunks in word 3 of the
+// 128-byte line ctl[kCtlLine (s + 1) ..].  Superblocks complete in order (each
+// folds its predecessor), so ctl[1] >= k means superblocks 0 .. k-1 are solved:
+// what workgroups whose turn is far off poll (one thread each); the next
+// superblock's workgroups poll their predecessor's solution itself.
+// tags: four arrays of n published values (2n words each): solution,
+// accumulated values, and for refined blocks first solution and residual.
 //
 // REFINE (FP64 factors): the inverse of an ill-conditioned 512 x 512
 // diagonal block applied to the accumulated values loses digits that a
@@ -345,14 +352,23 @@ __global__ void sbcond_kernel(int64_t nblk, const double* __restrict__ part, dou
 // the preconditioner need neither: an application error there only perturbs
 // the preconditioner.
 constexpr int kSweepThreads = 512;
+constexpr unsigned kTag = 1;         // tag of a published word (0: not yet)
+constexpr int64_t kTagWords = 8;     // tagged words per row: four arrays of two words
 constexpr int kSweepWaves = kSweepThreads / 64;
+// Orders a wave's LDS writes before its following LDS reads.
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <typename TF, bool FWD, bool TRANS, int WHICH, bool REFINE>
 __global__ __launch_bounds__(kSweepThreads) void sbsweep_kernel(const TF* __restrict__ F, int64_t lda, int64_t n,
                                                                 const double* __restrict__ D512,
                                                                 const double* __restrict__ dinv64,
                                                                 const double* __restrict__ cond, double* __restrict__ y,
-                                                                double* __restrict__ P, unsigned* __restrict__ ctl,
-                                                                uint64_t wait_ticks) {
+                                                                unsigned long long* __restrict__ tags,
+                                                                unsigned* __restrict__ ctl, uint64_t wait_ticks) {
   typedef double T;
   constexpr int RW = CH / kSweepWaves;        // chunk rows per wave (no-transpose)
   constexpr int NG = 2 * kSweepWaves;         // half-wave groups (transpose)
@@ -363,7 +379,8 @@ __global__ __launch_bounds__(kSweepThreads) void sbsweep_kernel(const TF* __rest
   __shared__ T xs2[SB];            // first solution, then its residual (REFINE)
   __shared__ T red[NG][CH + 1];    // cross-group partial sums
   __shared__ int s_t;
-  __shared__ unsigned s_avail, s_solved;
+  __shared__ unsigned s_solved;
+  __shared__ int s_failed;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t nsb = ceil_div(n, SB);
   unsigned* ticket = ctl;
@@ -371,7 +388,7 @@ __global__ __launch_bounds__(kSweepThreads) void sbsweep_kernel(const TF* __rest
   int* status = reinterpret_cast<int*>(ctl + 2);
   if (tid == 0) {
     s_t = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_avail = 0;
+    s_failed = 0;
     s_solved = 0;
     if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) s_t = INT_MAX;
   }
@@ -394,17 +411,19 @@ __global__ __launch_bounds__(kSweepThreads) void sbsweep_kernel(const TF* __rest
   //     columns]; reduced over the half-waves.
   const int tcol = lane & 31, tgrp = 2 * w + (lane >> 5);
 
-  // bounded wait of thread 0 until *ctr >= target; false if the solve failed.
-  // far: not on the critical path, poll less often
-  auto wait_count = [&](const unsigned* ctr, unsigned target, unsigned& v, bool far) -> bool {
+  // bounded polling of this thread; false if the solve failed.  far: not on
+  // the critical path, poll less often
+  auto wait_for = [&](auto&& ready, bool far) -> bool {
+    if (ready()) return true;
     uint32_t spins = 0;
     WaitClock clk(wait_ticks);
-    while ((v = ld_coh(ctr)) < target) {
+    for (;;) {
       if (far)
         __builtin_amdgcn_s_sleep(8);
       else
         __builtin_amdgcn_s_sleep(1);
       ++spins;
+      if (ready()) return true;
       if (clk.expired()) {
         __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return false;
@@ -412,7 +431,29 @@ __global__ __launch_bounds__(kSweepThreads) void sbsweep_kernel(const TF* __rest
       if ((spins & 255u) == 0 && __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
         return false;
     }
-    return true;
+  };
+  // published values: entry i of array e
+  auto publish = [&](int e, int64_t i, T v) {
+    unsigned long long* w2 = tags + 2 * (e * n + i);
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    st_coh(w2, (b << 32) | kTag);
+    st_coh(w2 + 1, (b & 0xFFFFFFFF00000000ull) | kTag);
+  };
+  auto published = [&](int e, int64_t i, T& v) -> bool {
+    const unsigned long long* w2 = tags + 2 * (e * n + i);
+    const unsigned long long lo = ld_coh(w2), hi = ld_coh(w2 + 1);
+    v = __longlong_as_double((long long)((hi & 0xFFFFFFFF00000000ull) | (lo >> 32)));
+    return (unsigned)lo == kTag && (unsigned)hi == kTag;
+  };
+  // stage the superblock's values of array e in dst (one per thread), waiting
+  // for each; ends with a barrier
+  static_assert(SB == kSweepThreads, "one published value per thread");
+  auto collect = [&](int e, int64_t o, int sz, T* dst) -> bool {
+    T v = T(0);
+    if (tid < sz && !wait_for([&]() { return published(e, o + tid, v); }, false)) s_failed = 1;
+    dst[tid] = v;
+    __syncthreads();
+    return s_failed == 0;
   };
   // reduce the per-thread partial sums of a product into red; after the
   // barrier, thread r < CH reads its row's value with row_value(r)
@@ -420,8 +461,7 @@ __global__ __launch_bounds__(kSweepThreads) void sbsweep_kernel(const TF* __rest
     if constexpr (!TRANS) {
 #pragma unroll
       for (int k = 0; k < RW; ++k) {
-        T v = ps[k];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        const T v = wave_sum(ps[k]);
         if (lane == 0) red[0][RW * w + k] = v;
       }
     } else {
@@ -544,26 +584,17 @@ __global__ __launch_bounds__(kSweepThreads) void sbsweep_kernel(const TF* __rest
     product(dv, vec, ps);
     reduce_rows(ps);
   };
-  // publish the chunk's CH values of stage e into buf, wait for the
-  // superblock's other chunks, then stage the superblock's SB values in dst
-  auto exchange = [&](T* buf, int e, T value, T* dst) -> bool {
-    if (tid < nr) st_coh(buf + oI + rc0 + tid, value);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (tid == 0) {
-      __hip_atomic_fetch_add(parts + e, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      unsigned v;
-      s_avail = wait_count(parts + e, (unsigned)NCH, v, false) ? 0u : 0xffffffffu;
-    }
-    __syncthreads();
-    if (s_avail == 0xffffffffu) return false;
-    for (int q = tid; q < SB; q += kSweepThreads) dst[q] = q < szI ? ld_coh(buf + oI + q) : T(0);
-    __syncthreads();
-    return true;
+  // publish the chunk's CH values into array e, start the loads that the next
+  // product needs (they overlap the trip, and the values leave first), then
+  // stage the superblock's SB values in dst
+  auto exchange = [&](int e, T value, T* dst, auto&& loads) -> bool {
+    if (tid < nr) publish(e, oI + rc0 + tid, value);
+    loads();
+    return collect(e, oI, szI, dst);
   };
 
   // 1. fold the superblocks solved before this one, in solve order.  The
-  // predecessor's completion is polled on its own line; earlier superblocks
+  // predecessor's solution is polled value by value; earlier superblocks
   // through the solved count, so a workgroup that starts late folds them
   // without a poll each.  FP32 factors leave room to hold the diagonal
   // inverse's rows during the last wait as well; FP64 ones load them after
@@ -582,61 +613,117 @@ __global__ __launch_bounds__(kSweepThreads) void sbsweep_kernel(const TF* __rest
     load_F(tv, oJ, szJ, false);
     if (kEarlyD && d == s - 1) load_D(dv);
     __syncthreads();  // xs free
-    if (tid == 0 && s_solved <= (unsigned)d) {
-      unsigned v;
-      bool ok;
-      if (d + 1 < s) {
-        ok = wait_count(solved, (unsigned)(d + 1), v, true);
-      } else {
-        ok = wait_count(ctl + kCtlLine * (d + 1) + 3, (unsigned)NCH, v, false);
-        v = d + 1;
+    if (d + 1 < s) {
+      if (tid == 0 && s_solved <= (unsigned)d) {
+        unsigned v = 0;
+        if (!wait_for([&]() { return (v = ld_coh(solved)) >= (unsigned)(d + 1); }, true)) s_failed = 1;
+        s_solved = v;
       }
-      s_solved = v;
-      s_avail = ok ? 0u : 0xffffffffu;
+      __syncthreads();
+      if (s_failed) return;
+      xs[tid] = tid < szJ ? ld_coh(y + oJ + tid) : T(0);  // complete: half the bytes of its tagged words
+      __syncthreads();
+    } else if (!collect(0, oJ, szJ, xs)) {
+      return;
     }
-    __syncthreads();
-    if (s_avail == 0xffffffffu) return;
-    for (int e = tid; e < SB; e += kSweepThreads) xs[e] = e < szJ ? ld_coh(y + oJ + e) : T(0);
-    __syncthreads();
     product(tv, xs, ps);
   }
-  if (!kEarlyD) load_D(dv);
   // 2. accumulated values b - (sum of the folded tiles); exchange them
   __syncthreads();
   reduce_rows(ps);
   __syncthreads();
   T acc_r = tid < nr ? y[oI + rc0 + tid] - row_value(tid) : T(0);
-  if (!exchange(P, 0, acc_r, xs)) return;
+  if (!exchange(1, acc_r, xs, [&]() {
+        if (!kEarlyD) load_D(dv);
+      }))
+    return;
   // 3. x = rows of D applied to the superblock's accumulated values
   T x;
   if constexpr (REFINE) {
     if (cond[I * 2 + WHICH] > kCondRobust) {
       // ill-conditioned block: every chunk solves the whole block by
       // substitution over its 64-row sub-blocks with their 64 x 64 inverses
-      // (xs: values still to solve, xs2: solution), then keeps its rows
+      // (xs: values still to solve, xs2: solution), then keeps its rows.  The
+      // next inverse, and the factor's entries four batches ahead, load while
+      // the ones before are used.  A thread adds a row's terms in order; its
+      // entries are coalesced in the transposed sweep, and in the other one
+      // pass through the wave's part of ds (8 columns of 64 rows at a time).
+      // 20-25 us a block; 60-95 us with every entry loaded when it was needed.
+      __shared__ T ds[TB * (TB + 1)];
+      constexpr int kBatch = TRANS ? 16 : 8, kAhead = TRANS ? 2 : 4;
       const int nsub = (szI + TB - 1) / TB;
+      T dreg[TB * TB / kSweepThreads];
+      auto load_inv = [&](int b) {
+        const double* D64 = dinv64 + ((I * (SB / TB) + b) * 2 + WHICH) * (int64_t)(TB * TB);
+#pragma unroll
+        for (int q = 0; q < TB * TB / kSweepThreads; ++q) dreg[q] = D64[tid + q * kSweepThreads];
+      };
+      TF ent[kAhead][kBatch];
+      // batch k of the columns of sub-block ob: this thread's row (TRANS), or
+      // rows 8 q + lane / 8 of the wave's 64, column lane % 8
+      auto load_batch = [&](int k, int ob, bool on) {
+#pragma unroll
+        for (int q = 0; q < kBatch; ++q) {
+          TF& v = ent[k % kAhead][q];
+          if constexpr (TRANS) {
+            const int64_t j = oI + ob + k * kBatch + q;
+            v = on && j < n && tid < szI ? F[j * lda + oI + tid] : TF(0);
+          } else {
+            const int64_t i = oI + 64 * w + 8 * q + (lane >> 3), j = oI + ob + k * kBatch + (lane & 7);
+            v = on && i < n && j < n ? F[i * lda + j] : TF(0);
+          }
+        }
+      };
+      load_inv(FWD ? 0 : nsub - 1);
       for (int st = 0; st < nsub; ++st) {
         const int b = FWD ? st : nsub - 1 - st;
         const int ob = b * TB;
-        const double* D64 = dinv64 + ((I * (SB / TB) + b) * 2 + WHICH) * (int64_t)(TB * TB);
+        const bool on = FWD ? w > b : w < b;  // (64 rows per wave: all of them or none)
+#pragma unroll
+        for (int q = 0; q < TB * TB / kSweepThreads; ++q) {
+          const int e = tid + q * kSweepThreads;
+          ds[e / TB * (TB + 1) + e % TB] = dreg[q];
+        }
+        if (st + 1 < nsub) load_inv(FWD ? b + 1 : b - 1);
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) load_batch(k, ob, on);
+        __syncthreads();
         if (tid < TB) {
           T a = 0;
+#pragma unroll 16
           for (int c2 = 0; c2 < TB; ++c2)
-            a = __builtin_fma(TRANS ? D64[c2 * TB + tid] : D64[tid * TB + c2], xs[ob + c2], a);
+            a = __builtin_fma(ds[TRANS ? c2 * (TB + 1) + tid : tid * (TB + 1) + c2], xs[ob + c2], a);
           xs2[ob + tid] = ob + tid < szI ? a : T(0);
         }
         __syncthreads();
-        const int cend = szI - ob < TB ? szI - ob : TB;
-        for (int i = tid; i < szI; i += kSweepThreads) {
-          if (FWD ? i >= ob + TB : i < ob) {
-            T a = 0;
-            for (int c2 = 0; c2 < cend; ++c2) {
-              const int64_t j = ob + c2;
-              const TF t = TRANS ? F[(oI + j) * lda + oI + i] : F[(oI + i) * lda + oI + j];
-              a = __builtin_fma((T)t, xs2[j], a);
+        if (on) {
+          const int cend = szI - ob < TB ? szI - ob : TB;
+          T* buf = ds + 64 * kBatch * w;
+          T a = 0;
+#pragma unroll
+          for (int k = 0; k < TB / kBatch; ++k) {
+            T v[kBatch];
+            if constexpr (TRANS) {
+#pragma unroll
+              for (int q = 0; q < kBatch; ++q) v[q] = (T)ent[k % kAhead][q];
+            } else {
+              // (the xor spreads the 32 lanes of an access over the banks)
+#pragma unroll
+              for (int q = 0; q < kBatch; ++q) {
+                const int r = 8 * q + (lane >> 3);
+                buf[r * 8 + ((lane & 7) ^ ((r >> 2) & 7))] = (T)ent[k % kAhead][q];
+              }
+              wave_fence();
+#pragma unroll
+              for (int q = 0; q < kBatch; ++q) v[q] = buf[lane * 8 + (q ^ ((lane >> 2) & 7))];
+              wave_fence();
             }
-            xs[i] -= a;
+            if (k + kAhead < TB / kBatch) load_batch(k + kAhead, ob, on);
+#pragma unroll
+            for (int q = 0; q < kBatch; ++q)
+              if (k * kBatch + q < cend) a = __builtin_fma(v[q], xs2[ob + k * kBatch + q], a);
           }
+          if (tid < szI) xs[tid] -= a;
         }
         __syncthreads();
       }
@@ -653,28 +740,27 @@ __global__ __launch_bounds__(kSweepThreads) void sbsweep_kernel(const TF* __rest
     // x0 exchanged; r = acc - T_KK x0 (or T_KK^T x0) on the chunk's rows;
     // exchanged; x += D r.  The diagonal tile loads during the first
     // exchange, D's rows again during the second.
-    T* X0 = P + n;
-    T* Rb = P + 2 * n;
     TF uv[NV];
-    load_F(uv, oI, szI, true);
-    if (!exchange(X0, 1, x, xs2)) return;
+    if (!exchange(2, x, xs2, [&]() { load_F(uv, oI, szI, true); })) return;
     T pr[NP];
 #pragma unroll
     for (int k = 0; k < NP; ++k) pr[k] = 0;
     product(uv, xs2, pr);
-    load_D(dv);
     __syncthreads();
     reduce_rows(pr);
     __syncthreads();
     // L_KK has a unit diagonal that is not stored: its x0 term
     const T r_r = tid < nr ? xs[rc0 + tid] - row_value(tid) - (WHICH == 0 ? xs2[rc0 + tid] : T(0)) : T(0);
-    if (!exchange(Rb, 2, r_r, xs2)) return;
+    if (!exchange(3, r_r, xs2, [&]() { load_D(dv); })) return;
     apply(dv, xs2);
     __syncthreads();
     if (tid < nr) x += row_value(tid);
   }
 publish:
-  if (tid < nr) st_coh(y + oI + rc0 + tid, x);
+  if (tid < nr) {
+    publish(0, oI + rc0 + tid, x);
+    st_coh(y + oI + rc0 + tid, x);
+  }
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (tid == 0) {
@@ -684,11 +770,14 @@ publish:
   }
 }
 
-// Clears the ticket and the superblocks' control lines; the solve's status
-// word ctl[2] stays.
-__global__ void reset_sweep_ctl_kernel(unsigned* ctl, int64_t nsb) {
+// Clears the ticket, the superblocks' control lines and the tags of the four
+// published arrays; the solve's status word ctl[2] stays.
+__global__ __launch_bounds__(256) void reset_sweep_kernel(unsigned* ctl, int64_t nsb, unsigned long long* tags,
+                                                          int64_t ntags) {
+  typedef unsigned long long vu2 __attribute__((ext_vector_type(2)));
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < 2 || (i >= kCtlLine && i < kCtlLine * (nsb + 1))) ctl[i] = 0u;
+  if (2 * i < ntags) reinterpret_cast<vu2*>(tags)[i] = vu2{0ull, 0ull};
 }
 
 // 64 x 64 inverses of L and U, then the 512 x 512 ones, then the condition
@@ -697,12 +786,13 @@ static int64_t dinv64_elems(int64_t n) { return ceil_div(n, TB) * 2 * TB * TB; }
 
 template <typename T>
 static int launch_sbsweep(bool fwd, bool trans, int which, const T* F, int64_t lda, int64_t n,
-                          const double* dinv, double* y, double* P, unsigned* ctl, hipStream_t s) {
+                          const double* dinv, double* y, unsigned long long* tags, unsigned* ctl, hipStream_t s) {
   const double* D512 = dinv + dinv64_elems(n);
   const double* cond = D512 + ceil_div(n, (int64_t)SB) * 2 * (int64_t)SB * SB;
   const int64_t nsb = ceil_div(n, (int64_t)SB);
-  hipLaunchKernelGGL(reset_sweep_ctl_kernel, dim3((unsigned)ceil_div(kCtlLine * (nsb + 1), 256)), dim3(256), 0, s,
-                     ctl, nsb);
+  hipLaunchKernelGGL(reset_sweep_kernel,
+                     dim3((unsigned)ceil_div(std::max<int64_t>(kCtlLine * (nsb + 1), kTagWords * n / 2), 256)), dim3(256),
+                     0, s, ctl, nsb, tags, kTagWords * n);
   RBFX_CHECK_LAUNCH();
   const uint64_t ticks = device_info().wait_ticks;
   const unsigned grid = (unsigned)(nsb * NCH);
@@ -711,7 +801,7 @@ static int launch_sbsweep(bool fwd, bool trans, int which, const T* F, int64_t l
   constexpr bool R64 = sizeof(T) == 8;
 #define RBFX_SBSWEEP(F_, T_, W_)                                                                              \
   hipLaunchKernelGGL((sbsweep_kernel<T, F_, T_, W_, R64>), dim3(grid), dim3(kSweepThreads), 0, s, F, \
-                     lda, n, D512, dinv, cond, y, P, ctl, ticks)
+                     lda, n, D512, dinv, cond, y, tags, ctl, ticks)
   if (fwd && !trans && which == 0) RBFX_SBSWEEP(true, false, 0);
   else if (!fwd && !trans && which == 1) RBFX_SBSWEEP(false, false, 1);
   else if (fwd && trans && which == 1) RBFX_SBSWEEP(true, true, 1);
@@ -726,32 +816,32 @@ static int launch_sbsweep(bool fwd, bool trans, int which, const T* F, int64_t l
   return RBFX_OK;
 }
 
-// Workspace of one solve: the permuted vector, the superblocks' accumulated
-// values, then the control words (3 + one per superblock).
+// Workspace of one solve: the permuted vector, the published values of a
+// sweep, then the control words (3 + one line per superblock).
 constexpr int64_t getrs_ctl_words(int64_t n) { return kCtlLine * ((n + SB - 1) / SB + 1) + 8; }
-// P holds three n-vectors: the accumulated values, and for the refined U
-// sweeps the first solutions and their residuals.
-static bool carve_getrs(void* work, size_t work_bytes, int64_t n, double*& y, double*& P, unsigned*& ctl) {
+static bool carve_getrs(void* work, size_t work_bytes, int64_t n, double*& y, unsigned long long*& tags,
+                        unsigned*& ctl) {
   Workspace ws(work, work_bytes);
   y = ws.take<double>(n);
-  P = ws.take<double>(3 * n);
+  tags = ws.take<unsigned long long>(kTagWords * n);
   ctl = ws.take<unsigned>(getrs_ctl_words(n));
-  return y && P && ctl;
+  return y && tags && ctl;
 }
 
-// The solve itself on carved scratch: y (n), P (3n), ctl (getrs_ctl_words).
+// The solve itself on carved scratch: y (n), tags (kTagWords n), ctl
+// (getrs_ctl_words).
 // Every scratch word that must start at zero is cleared by a kernel of the
 // solve (no memset), and nothing is allocated.
 template <typename T>
 static int getrs_run(int trans, int64_t n, const T* LU, int64_t lda, const int64_t* perm, const double* dinv,
-                     double* b, double* y, double* P, unsigned* ctl, hipStream_t s) {
+                     double* b, double* y, unsigned long long* tags, unsigned* ctl, hipStream_t s) {
   const unsigned g = (unsigned)ceil_div(n, 256);
   int st;
   if (!trans) {
     hipLaunchKernelGGL(gather_perm_kernel, dim3(g), dim3(256), 0, s, b, perm, n, y, ctl, 1);
     RBFX_CHECK_LAUNCH();
-    if ((st = launch_sbsweep<T>(true, false, 0, LU, lda, n, dinv, y, P, ctl, s))) return st;
-    if ((st = launch_sbsweep<T>(false, false, 1, LU, lda, n, dinv, y, P, ctl, s))) return st;
+    if ((st = launch_sbsweep<T>(true, false, 0, LU, lda, n, dinv, y, tags, ctl, s))) return st;
+    if ((st = launch_sbsweep<T>(false, false, 1, LU, lda, n, dinv, y, tags, ctl, s))) return st;
     hipLaunchKernelGGL(scatter_perm_kernel, dim3(g), dim3(256), 0, s, y, (const int64_t*)nullptr, n, b,
                        ctl);
     RBFX_CHECK_LAUNCH();
@@ -759,8 +849,8 @@ static int getrs_run(int trans, int64_t n, const T* LU, int64_t lda, const int64
     hipLaunchKernelGGL(gather_perm_kernel, dim3(g), dim3(256), 0, s, b, (const int64_t*)nullptr, n, y,
                        ctl, 1);
     RBFX_CHECK_LAUNCH();
-    if ((st = launch_sbsweep<T>(true, true, 1, LU, lda, n, dinv, y, P, ctl, s))) return st;
-    if ((st = launch_sbsweep<T>(false, true, 0, LU, lda, n, dinv, y, P, ctl, s))) return st;
+    if ((st = launch_sbsweep<T>(true, true, 1, LU, lda, n, dinv, y, tags, ctl, s))) return st;
+    if ((st = launch_sbsweep<T>(false, true, 0, LU, lda, n, dinv, y, tags, ctl, s))) return st;
     hipLaunchKernelGGL(scatter_perm_kernel, dim3(g), dim3(256), 0, s, y, perm, n, b, ctl);
     RBFX_CHECK_LAUNCH();
   }
@@ -772,10 +862,11 @@ static int getrs(int trans, int64_t n, const T* LU, int64_t lda, const int64_t* 
                  double* b, void* work, size_t work_bytes, hipStream_t s) {
   RBFX_REQUIRE(n > 0 && lda >= n && LU && perm && dinv && b, "bad getrs args");
   RBFX_REQUIRE(n < (int64_t)INT32_MAX / 2, "getrs: n too large");
-  double *y, *P;
+  double* y;
+  unsigned long long* tags;
   unsigned* ctl;
-  RBFX_REQUIRE(carve_getrs(work, work_bytes, n, y, P, ctl), "getrs workspace too small");
-  return getrs_run<T>(trans, n, LU, lda, perm, dinv, b, y, P, ctl, s);
+  RBFX_REQUIRE(carve_getrs(work, work_bytes, n, y, tags, ctl), "getrs workspace too small");
+  return getrs_run<T>(trans, n, LU, lda, perm, dinv, b, y, tags, ctl, s);
 }
 
 
@@ -854,9 +945,10 @@ static int getrs_multi(int64_t n, const double* LU, int64_t lda, const int64_t* 
 // Status of the last solve queued with this workspace (synchronises).
 static int getrs_status(int64_t n, void* work, size_t work_bytes, hipStream_t s) {
   RBFX_REQUIRE(n > 0 && work, "bad getrs_status args");
-  double *y, *P;
+  double* y;
+  unsigned long long* tags;
   unsigned* ctl;
-  RBFX_REQUIRE(carve_getrs(work, work_bytes, n, y, P, ctl), "getrs workspace too small");
+  RBFX_REQUIRE(carve_getrs(work, work_bytes, n, y, tags, ctl), "getrs workspace too small");
   unsigned st = 0;
   RBFX_HIP(hipMemcpyAsync(&st, ctl + 2, sizeof(st), hipMemcpyDeviceToHost, s));
   RBFX_HIP(hipStreamSynchronize(s));
@@ -921,7 +1013,7 @@ extern "C" int64_t rbfx_getrs_dinv_elems(int64_t n) {
 
 extern "C" size_t rbfx_getrs_workspace(int64_t n) {
   if (n <= 0) return 0;
-  return ws_round((size_t)n * sizeof(double)) + ws_round((size_t)3 * n * sizeof(double)) +
+  return ws_round((size_t)n * sizeof(double)) + ws_round((size_t)kTagWords * n * sizeof(unsigned long long)) +
          ws_round(getrs_ctl_words(n) * sizeof(unsigned)) + 512;
 }
 
@@ -950,11 +1042,11 @@ extern "C" int rbfx_getrs_f64(int trans, int64_t n, const double* d_LU, int64_t 
 namespace rbfx {
 // ---- allocation-free solve ------------------------------------------------------
 // Scratch of rbfx_getrs_noalloc_f64 for n <= RBFX_GETRS_NOALLOC_MAX_N, carved
-// like a getrs workspace: y (n doubles), P (3n doubles), control words.  One
+// like a getrs workspace: y (n doubles), published values, control words.  One
 // copy per device.  Host code never uses the symbol itself: its device
 // address comes from hipGetSymbolAddress, once per device.
 constexpr int64_t kNoAllocMaxN = RBFX_GETRS_NOALLOC_MAX_N;
-constexpr size_t kNoAllocBytes = 4 * (((size_t)kNoAllocMaxN * 8 + 255) / 256 * 256) +
+constexpr size_t kNoAllocBytes = (1 + kTagWords) * (((size_t)kNoAllocMaxN * 8 + 255) / 256 * 256) +
                                  ((size_t)getrs_ctl_words(kNoAllocMaxN) * 4 + 255) / 256 * 256;
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 static std::mutex g_scratch_mu;
@@ -984,10 +1076,11 @@ extern "C" int rbfx_getrs_noalloc_f64(int trans, int64_t n, const double* d_LU, 
   void* base = nullptr;
   int st;
   if ((st = scratch_address(base))) return st;
-  double *y, *P;
+  double* y;
+  unsigned long long* tags;
   unsigned* ctl;
-  RBFX_REQUIRE(carve_getrs(base, kNoAllocBytes, n, y, P, ctl), "solve scratch too small");
-  return getrs_run<double>(trans, n, d_LU, lda, d_perm, d_dinv, d_b, y, P, ctl, as_stream(stream));
+  RBFX_REQUIRE(carve_getrs(base, kNoAllocBytes, n, y, tags, ctl), "solve scratch too small");
+  return getrs_run<double>(trans, n, d_LU, lda, d_perm, d_dinv, d_b, y, tags, ctl, as_stream(stream));
 }
 
 extern "C" int rbfx_getrs_status(int64_t n, void* d_work, size_t work_bytes, void* stream) {
