@@ -139,7 +139,8 @@ int rbfx_matvec(const rbfx_problem* p, int matrix, int trans, const double* d_x,
  * coeffs = [lambda (N); gamma (M)].  All N centres are summed, the evaluation
  * point included (phi(0) for values, 0 for derivatives at r = 0).
  * Replaces updes/operators.py:118-150 (value/value_vec), 156-187
- * (gradient/gradient_vec) and 319-351 (laplacian/laplacian_vec).          */
+ * (gradient/gradient_vec) and 319-351 (laplacian/laplacian_vec).  Rows t not
+ * in ops_mask are not touched.                                            */
 int rbfx_eval(int kernel, double param, int64_t N, int64_t M, const double* d_cx,
               const double* d_cy, const double* d_coeffs, int64_t npts,
               const double* d_px, const double* d_py, uint32_t ops_mask,

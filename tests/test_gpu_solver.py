@@ -164,6 +164,38 @@ def test_eval_and_transpose_every_operator(kind, param, N, P):
         assert nan[P // 2] and nan.sum() == 1
 
 
+@pytest.mark.parametrize("kind,param", C.KINDS)
+@pytest.mark.parametrize("N,P", [(5, 1), (2049, 5), (33, 2047), (40, 2049)])
+def test_gradient_in_one_evaluation(kind, param, N, P):
+    """Both components in one kernel (one or four points per workgroup) against
+    the oracle's closed forms, with a point on a centre, a NaN point that stays
+    in its own row, and its adjoint against the transposes by component."""
+    from updes_amd import engine as E
+    from updes_amd.adjoint import EvalGrad
+    rng = np.random.default_rng(N + P)
+    ctr, pts = rng.uniform(0, 1, (N, 2)), rng.uniform(0, 1, (P, 2))
+    pts[0] = ctr[-1]
+    M = 6
+    c, w = rng.standard_normal(N + M), rng.standard_normal((P, 2))
+    ops = R.rbf_ops(kind, param, pts[:, :1], pts[:, 1:], ctr[None, :, 0], ctr[None, :, 1])
+    mon = np.stack([R.monomial_ops(m, pts[:, 0], pts[:, 1]) for m in range(M)], axis=-1)
+    full = np.concatenate([ops, mon], axis=2)[[R.DX, R.DY]]        # (2, P, N + M)
+    # |sum - exact| <= count eps sum |terms|, with the closed forms' own few eps
+    tol = 16 * np.finfo(float).eps * np.sqrt(N + P) * (np.abs(full) @ np.abs(c)).max(axis=1)
+    dctr, dpts, dw = (torch.as_tensor(v).cuda() for v in (ctr, pts, w))
+    dc = torch.as_tensor(c).cuda().requires_grad_(True)
+    g = EvalGrad.apply(dc, kind, param, dctr, dpts)
+    assert g.shape == (P, 2)
+    assert (np.abs(g.detach().cpu().numpy() - (full @ c).T).max(axis=0) <= tol).all()
+    (g * dw).sum().backward()
+    back = E.eval_t(kind, param, dctr, M, dpts, R.DX, dw[:, 0]) + E.eval_t(kind, param, dctr, M, dpts, R.DY, dw[:, 1])
+    assert torch.equal(dc.grad, back)
+    bad = dpts.clone()
+    bad[P // 2, 1] = float("nan")
+    nan = torch.isnan(EvalGrad.apply(dc.detach(), kind, param, dctr, bad)).cpu().numpy()
+    assert nan[P // 2].all() and nan.sum() == 2
+
+
 def test_integrate_field_matches_oracle_and_reference_test():
     """updes/tests/test_integrals.py on the GPU path: r^11, degree 3, 12 x 12,
     x^2/(1+y^2): same integral as the oracle, and |I - pi/12| < 0.1."""

@@ -71,12 +71,29 @@ class EvalOp(torch.autograd.Function):
     @staticmethod
     def forward(ctx, coeffs, kind, param, centers, points, op):
         ctx.save = (kind, param, centers, points, op, coeffs.numel() - centers.shape[0])
-        return E.eval_ops(kind, param, centers, coeffs, points, 1 << op)[op].clone()
+        return E.eval_rows(kind, param, centers, coeffs, points, op)[0]
 
     @staticmethod
     def backward(ctx, g):
         kind, param, centers, points, op, M = ctx.save
         return E.eval_t(kind, param, centers, M, points, op, g), None, None, None, None, None
+
+
+class EvalGrad(torch.autograd.Function):
+    """Gradient (P, 2) of the field ``coeffs`` at ``points``: both components
+    in one evaluation."""
+
+    @staticmethod
+    def forward(ctx, coeffs, kind, param, centers, points):
+        ctx.save = (kind, param, centers, points, coeffs.numel() - centers.shape[0])
+        return E.eval_rows(kind, param, centers, coeffs, points, L.DX, 2).t().contiguous()
+
+    @staticmethod
+    def backward(ctx, g):
+        kind, param, centers, points, M = ctx.save
+        w = g.t().contiguous()
+        out = E.eval_t(kind, param, centers, M, points, L.DX, w[0])
+        return out.add_(E.eval_t(kind, param, centers, M, points, L.DY, w[1])), None, None, None, None
 
 
 class RhsAssemble(torch.autograd.Function):

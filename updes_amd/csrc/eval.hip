@@ -16,9 +16,9 @@ constexpr int kEvPts = 4;
 // usual call (value, one component of the gradient, the Laplacian): the
 // kernel then forms that operator alone, with r from the square-root
 // sequence without range scaling where every r^2 of the wave allows it (the
-// same bits as sqrt; NaN and extreme distances take sqrt itself).  kSetAll
-// forms all seven.
-enum OpSet { kSetVal = 0, kSetGrad = 1, kSetLap = 2, kSetAll = 3 };
+// same bits as sqrt; NaN and extreme distances take sqrt itself).  kSetBoth is
+// both components of the gradient from one square root, kSetAll all seven.
+enum OpSet { kSetVal = 0, kSetGrad = 1, kSetLap = 2, kSetAll = 3, kSetBoth = 4 };
 
 __host__ inline int op_set(uint32_t mask) {
   switch (mask) {
@@ -26,6 +26,7 @@ __host__ inline int op_set(uint32_t mask) {
     case 1u << RBFX_DX:
     case 1u << RBFX_DY: return kSetGrad;
     case 1u << RBFX_LAP: return kSetLap;
+    case (1u << RBFX_DX) | (1u << RBFX_DY): return kSetBoth;
     default: return kSetAll;
   }
 }
@@ -129,6 +130,68 @@ __global__ __launch_bounds__(kEvThreads) void eval_op_kernel(Kern k, int64_t N, 
       s += coeffs[N + m] * o[op];
     }
     out[(int64_t)op * npts + p0 + q] = s;
+  }
+}
+
+// Both components of the gradient (the same sums) from one square root: 0.43 ms
+// at 40,007 points and 10,000 centres (r^3), two kernels of one component 0.92 ms;
+// at 33 points of 600 centres one launch of 13 us instead of two.
+template <int KIND, bool FAST, int PTS>
+__global__ __launch_bounds__(kEvThreads) void eval_grad_kernel(Kern k, int64_t N, int64_t M,
+                                                               const double* __restrict__ cx,
+                                                               const double* __restrict__ cy,
+                                                               const double* __restrict__ coeffs, int64_t npts,
+                                                               const double* __restrict__ px,
+                                                               const double* __restrict__ py,
+                                                               double* __restrict__ out) {
+  pin_kind<KIND, FAST>(k);
+  const int64_t p0 = (int64_t)blockIdx.x * PTS;
+  double xp[PTS], yp[PTS], acc[2 * PTS];
+#pragma unroll
+  for (int q = 0; q < PTS; ++q) {
+    const int64_t p = p0 + q < npts ? p0 + q : npts - 1;
+    xp[q] = px[p];
+    yp[q] = py[p];
+    acc[q] = acc[PTS + q] = 0.0;
+  }
+  for (int64_t j = threadIdx.x; j < N; j += kEvThreads) {
+    const double wj = coeffs[j], xj = cx[j], yj = cy[j];
+    double dx[PTS], dy[PTS], r[PTS];
+    bool mid = true;
+#pragma unroll
+    for (int q = 0; q < PTS; ++q) {
+      dx[q] = xp[q] - xj;
+      dy[q] = yp[q] - yj;
+      r[q] = dist2(dx[q], dy[q]);
+      mid = mid && mid_or_zero(r[q]);
+    }
+    if (__all(mid)) {
+#pragma unroll
+      for (int q = 0; q < PTS; ++q) r[q] = r[q] > 0.0 ? sqrt_mid(r[q]) : 0.0;
+    } else {
+#pragma unroll
+      for (int q = 0; q < PTS; ++q) r[q] = sqrt(r[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < PTS; ++q) {
+      acc[q] += wj * pair_op<kSetGrad>(k, r[q], dx[q]);
+      acc[PTS + q] += wj * pair_op<kSetGrad>(k, r[q], dy[q]);
+    }
+  }
+  __shared__ double red[2 * PTS][kEvThreads / 64];
+  block_sums(acc, red);
+  if (threadIdx.x < 2 * PTS) {
+    const int q = threadIdx.x % PTS, op = threadIdx.x < PTS ? RBFX_DX : RBFX_DY;
+    const int64_t p = p0 + q;
+    if (p >= npts) return;
+    double s = 0.0;
+    for (int w = 0; w < kEvThreads / 64; ++w) s += red[threadIdx.x][w];
+    for (int64_t m = 0; m < M; ++m) {
+      double o[RBFX_NOPS];
+      mono_ops((int)m, px[p], py[p], o);
+      s += coeffs[N + m] * o[op];
+    }
+    out[(int64_t)op * npts + p] = s;
   }
 }
 
@@ -387,6 +450,14 @@ static int eval_launch(const Kern& k, int64_t N, int64_t M, const double* cx, co
       case kSetVal: RBFX_EVAL(kSetVal); break;
       case kSetGrad: RBFX_EVAL(kSetGrad); break;
       case kSetLap: RBFX_EVAL(kSetLap); break;
+      case kSetBoth:
+        if (four)
+          hipLaunchKernelGGL((eval_grad_kernel<KIND_, FAST_, kEvPts>), dim3(g4), dim3(kEvThreads), 0, s, k, N, M, cx,
+                             cy, coeffs, npts, px, py, out);
+        else
+          hipLaunchKernelGGL((eval_grad_kernel<KIND_, FAST_, 1>), dim3(g1), dim3(kEvThreads), 0, s, k, N, M, cx, cy,
+                             coeffs, npts, px, py, out);
+        break;
       default:
         hipLaunchKernelGGL((eval_all_kernel<KIND_, FAST_>), dim3(g4), dim3(kEvThreads), 0, s, k, N, M, cx, cy, coeffs,
                            npts, px, py, mask, out);

@@ -236,29 +236,43 @@ def matvec(problem, x, matrix=L.MAT_K, trans=False):
     return y
 
 
+def _xy(points):
+    """Contiguous x and y of (P, 2) points, from one copy."""
+    t = points.detach().to(torch.float64).reshape(-1, 2).t().contiguous()
+    return t[0], t[1]
+
+
+def _eval_into(kind, param, centers, coeffs, points, mask, out, first):
+    """rbfx_eval of the operators of mask into out, whose first row is operator ``first``."""
+    cx, cy = _xy(centers)
+    px, py = _xy(points)
+    coeffs = coeffs.detach().to(torch.float64).contiguous()
+    N, P = cx.numel(), px.numel()
+    if P:
+        # the library writes operator t at row t: rows before `first` are not
+        # in the mask and not touched
+        base = ctypes.c_void_p(out.data_ptr() - 8 * first * P)
+        L.check(L.lib().rbfx_eval(int(kind), float(param), N, coeffs.numel() - N, L.ptr(cx), L.ptr(cy), L.ptr(coeffs),
+                                  P, L.ptr(px), L.ptr(py), int(mask), base, L.stream()))
+    return out
+
+
 def eval_ops(kind, param, centers, coeffs, points, mask):
     """(7, P) operator values of the field ``coeffs`` at ``points`` (rows of mask set)."""
-    centers = centers.detach().to(torch.float64)
-    cx, cy = centers[:, 0].contiguous(), centers[:, 1].contiguous()
-    pts = points.detach().to(torch.float64).reshape(-1, 2)
-    px, py = pts[:, 0].contiguous(), pts[:, 1].contiguous()
-    coeffs = coeffs.detach().to(torch.float64).contiguous()
-    N = cx.numel()
-    M = coeffs.numel() - N
-    P = px.numel()
-    out = torch.zeros((L.NOPS, P), dtype=torch.float64, device=cx.device)
-    if P:
-        L.check(L.lib().rbfx_eval(int(kind), float(param), N, M, L.ptr(cx), L.ptr(cy), L.ptr(coeffs), P,
-                                  L.ptr(px), L.ptr(py), int(mask), L.ptr(out), L.stream()))
-    return out
+    out = torch.zeros((L.NOPS, points.numel() // 2), dtype=torch.float64, device=centers.device)
+    return _eval_into(kind, param, centers, coeffs, points, mask, out, 0)
+
+
+def eval_rows(kind, param, centers, coeffs, points, op, count=1):
+    """(count, P) values of the operators op .. op + count - 1 alone."""
+    out = torch.empty((count, points.numel() // 2), dtype=torch.float64, device=centers.device)
+    return _eval_into(kind, param, centers, coeffs, points, ((1 << count) - 1) << op, out, op)
 
 
 def eval_t(kind, param, centers, M, points, op, w):
     """Adjoint of eval_ops for one operator: (N+M,) vector."""
-    centers = centers.detach().to(torch.float64)
-    cx, cy = centers[:, 0].contiguous(), centers[:, 1].contiguous()
-    pts = points.detach().to(torch.float64).reshape(-1, 2)
-    px, py = pts[:, 0].contiguous(), pts[:, 1].contiguous()
+    cx, cy = _xy(centers)
+    px, py = _xy(points)
     w = w.detach().to(torch.float64).contiguous()
     N = cx.numel()
     out = torch.empty(N + int(M), dtype=torch.float64, device=cx.device)

@@ -143,7 +143,8 @@ def nodal_div_grad(x, center=None, rbf=None, monomial=None, args=None):
 
 # ---- field evaluation (operators.py:118-371) ----------------------------------
 def _eval_points(x):
-    """Points as (P, 2) and a function restoring the caller's layout."""
+    """Points as (P, 2) and a function restoring the caller's layout of
+    per-point results."""
     x = torch.as_tensor(x, dtype=torch.float64)
     if _TRACE[0] and x.dim() == 2 and x.shape[0] == 2:
         return x.T, (lambda v: v)            # vectorised trace: x is (2, rows)
@@ -153,6 +154,7 @@ def _eval_points(x):
 
 
 def _field_eval(x, field, centers, rbf, op):
+    """Operator ``op`` of a field at x, or with op None its gradient."""
     kind, param = rbf_spec(rbf)
     if isinstance(field, CoeffRef):
         return EvalExpr({(op, field.k): 1.0})
@@ -161,6 +163,8 @@ def _field_eval(x, field, centers, rbf, op):
     dev = torch.device("cuda")
     field = torch.as_tensor(field, dtype=torch.float64).to(dev)
     centers = torch.as_tensor(centers, dtype=torch.float64).to(dev)
+    if op is None:
+        return back(AD.EvalGrad.apply(field, kind, param, centers, pts.to(dev)))
     return back(AD.EvalOp.apply(field, kind, param, centers, pts.to(dev), op))
 
 
@@ -176,11 +180,9 @@ def value_vec(x, field, centers, rbf=None):
 
 def gradient(x, field, centers, rbf=None, clip_val=None):
     """Field gradient at x (``operators.py:156-184``)."""
-    gx = _field_eval(x, field, centers, rbf, L.DX)
-    gy = _field_eval(x, field, centers, rbf, L.DY)
-    if isinstance(gx, EvalExpr):
-        return EvalVec(gx, gy)
-    g = torch.stack([gx, gy], dim=-1)
+    if isinstance(field, CoeffRef):
+        return EvalVec(_field_eval(x, field, centers, rbf, L.DX), _field_eval(x, field, centers, rbf, L.DY))
+    g = _field_eval(x, field, centers, rbf, None)
     return torch.clamp(g, -clip_val, clip_val) if clip_val else g
 
 
