@@ -131,6 +131,47 @@ def test_gmres_ir_cardinal_matches_fp64_lu(trans):
     assert eta <= 2.0 ** -53, eta
 
 
+@pytest.mark.parametrize("nx,ny,M", [(12, 11, 3), (33, 31, 6), (52, 41, 3)])
+def test_cardinal_map_of_every_node(nx, ny, M):
+    """The map from cardinal to RBF coefficients against NumPy, special points
+    (in every stencil: fewer, and more, occurrences than one workgroup has
+    threads) included: one iteration of GMRES returns a multiple of the
+    preconditioned right-hand side z = C K~^-1 v + P s."""
+    from updes_amd import engine as E
+    from updes_amd import _lib as L
+    ft = {"North": "d", "South": "d", "East": "d", "West": "d"}
+    oc, uc, prob, basis = _setup(R.POLYHARMONIC, 1.0, M, nx=nx, ny=ny, facets=ft, seed=2)
+    fac = E.KFactor(prob, "fp32_ir", basis=basis)
+    assert fac.mode == "cardinal"
+    N, lu = oc.N, fac.lu32
+    b = torch.as_tensor(np.random.default_rng(nx).standard_normal(N + M), device="cuda")
+    x = torch.empty_like(b)
+    ws = L.workspace(L.lib().rbfx_gmres_ir_cardinal_workspace(N, M, 1), "cuda")
+    c, stats = basis.struct(fac.rs), L.IrStats()
+    status = L.lib().rbfx_gmres_ir_cardinal(0, ctypes.byref(c), L.ptr(fac.K64), fac.K64.shape[1], 0.0, L.ptr(lu.a),
+                                            lu.ld, L.ptr(lu.perm), L.ptr(lu.dinv), L.ptr(b), L.ptr(x), 1e-30, 1, 1,
+                                            L.ptr(ws), ws.numel(), ctypes.byref(stats), L.stream())
+    assert status == L.RBFX_ERR_STALL and stats.inner_iters == 1
+    bs = b.clone()
+    bs[:N] *= fac.rs
+    v = bs / bs.norm()
+    t = lu.solve(v[:N]).cpu().numpy()
+    st = basis.stencil.cpu().numpy().reshape(N, basis.k)
+    Cm = CR.basis_matrix(st, basis.beta.cpu().numpy().reshape(N, basis.k),
+                         basis.alpha.cpu().numpy()[:N * M].reshape(N, M))
+    P = np.stack([R.monomial_ops(m, oc.sorted_nodes[:, 0], oc.sorted_nodes[:, 1])[R.VAL] for m in range(M)], axis=-1)
+    s = basis.ptp_inv.cpu().numpy().reshape(M, M) @ v[N:].cpu().numpy()
+    ref = Cm @ t
+    ref[:N] += P @ s
+    size = np.abs(Cm) @ np.abs(t)
+    size[:N] += np.abs(P) @ np.abs(s)
+    got = x.cpu().numpy()
+    scale = (got @ ref) / (ref @ ref)
+    # sums of at most N + M terms of entries that carry eps times the condition
+    # of K~ (below 1e5 at these sizes)
+    assert np.abs(got / scale - ref).max() <= 1e5 * np.finfo(float).eps * size.max()
+
+
 def test_cardinal_basis_rejects_bad_stencils():
     from updes_amd import engine as E, _lib as L
     oc, uc, prob, basis = _setup(R.POLYHARMONIC, 1.0, 3)

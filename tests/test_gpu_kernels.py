@@ -43,6 +43,29 @@ def test_gemv_matches_numpy(trans, m, n, lda, alpha, beta):
     assert np.abs(got - ref).max() <= 1e-14 * scale * max(1, (m if trans else n) ** 0.5)
 
 
+@pytest.mark.parametrize("m", [1, 3, 4, 31, 32, 33, 63, 64, 65])
+@pytest.mark.parametrize("n,lda,beta", [(1, 1, 0.0), (63, 64, 1.0), (65, 65, 0.0), (4097, 4100, -0.5)])
+def test_gemv_transposed_few_rows(m, n, lda, beta):
+    """Transposed product of at most 64 rows (one kernel, a wave per fourth
+    row) and of 65: against NumPy in FP64; y is not read when beta is 0, and an
+    infinite last row stays infinite."""
+    L = _lib()
+    rng = np.random.default_rng(m + 3 * n)
+    A, x, y0 = rng.standard_normal((m, lda)), rng.standard_normal(m), rng.standard_normal(n)
+    A[-1, 0], x[-1] = np.inf, 1.0
+    dA, dx = torch.as_tensor(A).cuda(), torch.as_tensor(x).cuda()
+    dy = torch.as_tensor(y0 if beta else np.full(n, np.nan)).cuda()
+    ws = L.workspace(L.lib().rbfx_gemv_workspace(1, m, n), "cuda")
+    L.check(L.lib().rbfx_gemv_f64(1, m, n, -1.0, L.ptr(dA), lda, L.ptr(dx), beta, L.ptr(dy), L.ptr(ws), ws.numel(),
+                                  L.stream()))
+    got = dy.cpu().numpy()
+    assert got[0] == -np.inf
+    ref = -(A[:, 1:n].T @ x) + (beta * y0[1:] if beta else 0.0)
+    # m products and m + 1 sums, each within eps / 2 of the terms' magnitudes, on both sides
+    bound = (m + 2) * np.finfo(float).eps * (np.abs(A[:, 1:n]).T @ np.abs(x) + np.abs(beta * y0[1:]))
+    assert (np.abs(got[1:] - ref) <= bound).all()
+
+
 @pytest.mark.parametrize("m,n,lda,nrs", [(1, 1, 1, 1), (300, 257, 264, 200), (5000, 301, 301, 5000), (64, 64, 64, 0)])
 def test_frobenius_norms_match_numpy(m, n, lda, nrs):
     """rbfx_frobenius_f64 (rows i < n_scaled scaled) and the one-pass pair

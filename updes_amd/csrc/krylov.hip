@@ -164,6 +164,47 @@ __global__ void gemv_t_finish_kernel(int64_t n, int64_t chunks, const double* __
   y[j] = alpha * s + (beta != 0.0 ? beta * y[j] : 0.0);
 }
 
+// The same for at most kGvFewRows rows (combinations of the basis vectors of
+// GMRES), whole: a workgroup takes 64 columns, wave w their rows w, w + 4, ...
+// with eight loads in flight a thread, and writes y itself.  Bound by latency:
+// 4 us for 2 to 4 rows of 10,006 columns, the chunks above and their finish 40 us
+// (79 workgroups that walk the rows one load at a time).  At 64 rows a chunk of
+// the kernel above fills its eight loads as well.
+constexpr int64_t kGvFewRows = 64;
+__global__ __launch_bounds__(kGvThreads) void gemv_t_few_kernel(int64_t m, int64_t n, double alpha,
+                                                                const double* __restrict__ A, int64_t lda,
+                                                                const double* __restrict__ x, double beta,
+                                                                double* __restrict__ y) {
+  constexpr int kWaves = kGvThreads / 64, kBatch = 8;
+  __shared__ double red[kWaves][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t j = (int64_t)blockIdx.x * 64 + lane, jc = j < n ? j : n - 1;
+  const double y0 = beta != 0.0 ? y[jc] : 0.0;
+  double s = 0.0;
+  for (int64_t i0 = w; i0 < m; i0 += kWaves * kBatch) {
+    double a[kBatch], xv[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int64_t i = i0 + kWaves * u < m ? i0 + kWaves * u : m - 1;
+      a[u] = A[i * lda + jc];
+      xv[u] = x[i];
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const double t = __builtin_fma(a[u], xv[u], s);
+      s = i0 + kWaves * u < m ? t : s;
+    }
+  }
+  red[w][lane] = s;
+  __syncthreads();
+  if (w == 0 && j < n) {
+    double t = red[0][lane];
+#pragma unroll
+    for (int q = 1; q < kWaves; ++q) t += red[q][lane];
+    y[j] = alpha * t + (beta != 0.0 ? beta * y0 : 0.0);
+  }
+}
+
 // Row chunks of the transposed product: about eight workgroups per CU.
 static int64_t gemv_t_chunks(int64_t m, int64_t n) {
   const int64_t colb = ceil_div(n, kGvTCols);
@@ -207,10 +248,16 @@ int gemv_launch(int trans, int64_t m, int64_t n, double alpha, const double* A, 
     RBFX_CHECK_LAUNCH();
     return RBFX_OK;
   }
+  RBFX_REQUIRE(part != nullptr, "gemv^T needs a workspace");
+  if (m <= kGvFewRows) {
+    hipLaunchKernelGGL(gemv_t_few_kernel, dim3((unsigned)ceil_div(n, 64)), dim3(kGvThreads), 0, s, m, n, alpha, A,
+                       lda, x, beta, y);
+    RBFX_CHECK_LAUNCH();
+    return RBFX_OK;
+  }
   const int64_t chunks = gemv_t_chunks(m, n);
   const int64_t rpc = ceil_div(m, chunks);
   const int64_t used = ceil_div(m, rpc);
-  RBFX_REQUIRE(part != nullptr, "gemv^T needs a workspace");
   hipLaunchKernelGGL(gemv_t_kernel, dim3((unsigned)ceil_div(n, kGvTCols), (unsigned)used), dim3(kGvThreads),
                      0, s, m, n, A, lda, x, rpc, part);
   RBFX_CHECK_LAUNCH();
