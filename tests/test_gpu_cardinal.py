@@ -172,6 +172,31 @@ def test_cardinal_map_of_every_node(nx, ny, M):
     assert np.abs(got / scale - ref).max() <= 1e5 * np.finfo(float).eps * size.max()
 
 
+def test_expired_sweep_wait_ends_the_refinement():
+    """A sweep whose wait expired (bound of 0 set from the host, at a size where
+    the factors' own solve runs into it) inside GMRES raises RBFX_ERR_TIMEOUT
+    in that iteration, not a stall and not a fallback; with the default bound
+    restored the same factors solve."""
+    import updes_amd as u
+    from updes_amd import engine as E
+    from updes_amd import _lib as L
+    ft = {"North": "d", "South": "d", "East": "d", "West": "d"}
+    uc = u.SquareCloud(Nx=142, Ny=141, facet_types=ft, jitter=C.jitter(142, 141, 0.2, 2))
+    prob = E.Problem(E.device_cloud(uc), R.POLYHARMONIC, 1.0, 3, E.OpDesc.builtin(3))
+    fac = E.KFactor(prob, "fp32_ir")
+    b = torch.as_tensor(np.random.default_rng(3).standard_normal(prob.n), device="cuda")
+    L.check(L.lib().rbfx_set_wait_seconds(0.0))
+    try:
+        for solve in (lambda: fac.lu32.solve(b[:prob.n - 3]), lambda: fac.solve(b), lambda: fac.solve(b, trans=True)):
+            with pytest.raises(L.RbfxError) as ei:
+                solve()
+            assert ei.value.status == L.RBFX_ERR_TIMEOUT
+    finally:
+        L.check(L.lib().rbfx_set_wait_seconds(-1.0))
+    assert torch.isfinite(fac.solve(b)).all() and not fac.last_stats.fell_back
+    assert torch.isfinite(fac.solve(b, trans=True)).all() and not fac.last_stats.fell_back
+
+
 def test_cardinal_basis_rejects_bad_stencils():
     from updes_amd import engine as E, _lib as L
     oc, uc, prob, basis = _setup(R.POLYHARMONIC, 1.0, 3)

@@ -865,10 +865,10 @@ struct CardPair : PairOp {
   hipStream_t s;
 
   int solve32(int tr) {
-    int st = rbfx_getrs_f32(tr, a.N, LU32, ld32, perm, dinv, t, ts_work, ts_bytes, s);
-    if (st) return st;
-    return rbfx_getrs_status(a.N, ts_work, ts_bytes, s);
+    return rbfx_getrs_f32(tr, a.N, LU32, ld32, perm, dinv, t, ts_work, ts_bytes, s);
   }
+  const unsigned* failed() override { return getrs_failed(a.N, ts_work, ts_bytes); }
+  int status() override { return rbfx_getrs_status(a.N, ts_work, ts_bytes, s); }
   int apply(const double* v, double* z, double* w) override {
     const unsigned gN = (unsigned)ceil_div(a.N, 256);
     double* part = red;

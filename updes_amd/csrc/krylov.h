@@ -11,7 +11,16 @@ namespace rbfx {
 struct PairOp {
   virtual ~PairOp() = default;
   virtual int apply(const double* v, double* z, double* w) = 0;
+  // Device word that is nonzero once the last apply failed (a bounded wait of
+  // its triangular sweeps expired, the result is NaN): read with the scalars
+  // of the iteration, then status() reports the error.
+  virtual const unsigned* failed() = 0;
+  virtual int status() = 0;
 };
+
+// Device word that a solve queued with this workspace (rbfx_getrs_*) sets when
+// it fails.
+const unsigned* getrs_failed(int64_t n, void* work, size_t work_bytes);
 
 // w = op(K) x in FP64 (the residual operator of the refinement).
 struct ResidualOp {

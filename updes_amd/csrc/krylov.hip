@@ -167,9 +167,10 @@ __global__ void gemv_t_finish_kernel(int64_t n, int64_t chunks, const double* __
 // The same for at most kGvFewRows rows (combinations of the basis vectors of
 // GMRES), whole: a workgroup takes 64 columns, wave w their rows w, w + 4, ...
 // with eight loads in flight a thread, and writes y itself.  Bound by latency:
-// 4 us for 2 to 4 rows of 10,006 columns, the chunks above and their finish 40 us
-// (79 workgroups that walk the rows one load at a time).  At 64 rows a chunk of
-// the kernel above fills its eight loads as well.
+// inside GMRES 4 us for 2 to 4 rows of 10,006 columns, the chunks above and their
+// finish 40 us; back to back on resident rows 8.4 to 9.5 us against 11.1 to 11.8 at
+// every number of rows from 1 to 64 and 600 to 40,006 columns (two launches
+// against one), past which the chunks share the work.
 constexpr int64_t kGvFewRows = 64;
 __global__ __launch_bounds__(kGvThreads) void gemv_t_few_kernel(int64_t m, int64_t n, double alpha,
                                                                 const double* __restrict__ A, int64_t lda,
@@ -282,8 +283,9 @@ __global__ __launch_bounds__(256) void dot_partial_kernel(int64_t n, const doubl
   __syncthreads();
   if (threadIdx.x == 0) part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
+// (and out[1] = 1 when the word `failed`, if given, is set, else 0)
 __global__ __launch_bounds__(256) void dot_final_kernel(int nparts, const double* __restrict__ part,
-                                                        double* __restrict__ out) {
+                                                        double* __restrict__ out, const unsigned* failed) {
   double s = 0.0;
   for (int i = threadIdx.x; i < nparts; i += 256) s += part[i];
   __shared__ double red[4];
@@ -291,6 +293,7 @@ __global__ __launch_bounds__(256) void dot_final_kernel(int nparts, const double
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
   if (threadIdx.x == 0) *out = red[0] + red[1] + red[2] + red[3];
+  if (threadIdx.x == 0 && failed) out[1] = *failed != 0u ? 1.0 : 0.0;
 }
 
 // y = a*x + b*y
@@ -348,10 +351,11 @@ __global__ __launch_bounds__(256) void fro_partial_kernel(int64_t m, int64_t n, 
   }
 }
 
-static int dot(int64_t n, const double* a, const double* b, double* part, double* out, hipStream_t s) {
+static int dot(int64_t n, const double* a, const double* b, double* part, double* out, hipStream_t s,
+               const unsigned* failed = nullptr) {
   hipLaunchKernelGGL(dot_partial_kernel, dim3(kDotBlocks), dim3(256), 0, s, n, a, b, part);
   RBFX_CHECK_LAUNCH();
-  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(256), 0, s, kDotBlocks, part, out);
+  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(256), 0, s, kDotBlocks, part, out, failed);
   RBFX_CHECK_LAUNCH();
   return RBFX_OK;
 }
@@ -551,9 +555,12 @@ int fgmres_ir(PairOp& pre, ResidualOp& res, int64_t n, const double* d_b, double
       if ((st = gemv(1, k + 1, n, -1.0, V, n, h1, 1.0, w, part, s))) return st;
       if ((st = gemv(0, k + 1, n, 1.0, V, n, w, 0.0, h2, nullptr, s))) return st;
       if ((st = gemv(1, k + 1, n, -1.0, V, n, h2, 1.0, w, part, s))) return st;
-      if ((st = dot(n, w, w, dpart, hd + 2 * m + 4, s))) return st;
+      if ((st = dot(n, w, w, dpart, hd + 2 * m + 4, s, pre.failed()))) return st;
       RBFX_HIP(hipMemcpyAsync(hh.data(), hd, (2 * m + 6) * sizeof(double), hipMemcpyDeviceToHost, s));
       RBFX_HIP(hipStreamSynchronize(s));
+      // (one synchronisation per iteration: a copy of the sweeps' status of its
+      // own left the device idle for 45 us)
+      if (hh[2 * m + 5] != 0.0 && (st = pre.status())) return st;
       const double hn = sqrt(hh[2 * m + 4]);
       for (int i = 0; i <= k; ++i) col[i] = hh[i] + hh[m + 1 + i];
       col[k + 1] = hn;
@@ -660,9 +667,10 @@ struct LuPair : PairOp {
     RBFX_CHECK_LAUNCH();
     int st = rbfx_getrs_f32(trans, n, LU32, ld32, perm, dinv, z, ts_work, ts_bytes, s);
     if (st) return st;
-    if ((st = rbfx_getrs_status(n, ts_work, ts_bytes, s))) return st;
     return K->applyK(z, w);
   }
+  const unsigned* failed() override { return getrs_failed(n, ts_work, ts_bytes); }
+  int status() override { return rbfx_getrs_status(n, ts_work, ts_bytes, s); }
 };
 
 size_t residual_ws_bytes(int64_t n) {

@@ -942,6 +942,14 @@ static int getrs_multi(int64_t n, const double* LU, int64_t lda, const int64_t* 
   return RBFX_OK;
 }
 
+// Device word that a solve queued with this workspace sets when it fails.
+const unsigned* getrs_failed(int64_t n, void* work, size_t work_bytes) {
+  double* y;
+  unsigned long long* tags;
+  unsigned* ctl;
+  return carve_getrs(work, work_bytes, n, y, tags, ctl) ? ctl + 2 : nullptr;
+}
+
 // Status of the last solve queued with this workspace (synchronises).
 static int getrs_status(int64_t n, void* work, size_t work_bytes, hipStream_t s) {
   RBFX_REQUIRE(n > 0 && work, "bad getrs_status args");
