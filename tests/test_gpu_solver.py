@@ -164,6 +164,40 @@ def test_eval_and_transpose_every_operator(kind, param, N, P):
         assert nan[P // 2] and nan.sum() == 1
 
 
+@pytest.mark.parametrize("kind", [R.POLYHARMONIC, R.THIN_PLATE])
+@pytest.mark.parametrize("param", [1.5, 2.0, 2.25, 2.5, 5.0, 7.5, 8.0, 8.5])
+def test_radial_powers(kind, param):
+    """r^(2a+1) and r^(2a) log r at one centre, where the exponent is whole
+    (products, up to 16) and where it is not or larger (pow), at ordinary and at
+    extreme distances, against extended precision."""
+    from updes_amd import engine as E
+    m = 2 * param + (1 if kind == R.POLYHARMONIC else 0)
+    rng = np.random.default_rng(int(8 * param) + kind)
+    top = min(1000.0 / m, 100.0)
+    r = 2.0 ** np.concatenate([rng.uniform(-3, 3, 500), rng.uniform(-top, top, 200), [59.9, 60.0, 60.1, -60.1]])
+    r = r[np.abs(m * np.log2(r)) < 1000]
+    r = np.concatenate([r, [0.0, 1e300, 1e-300, np.nan]])
+    pts = torch.zeros((r.size, 2), dtype=torch.float64, device="cuda")
+    pts[:, 0] = torch.as_tensor(r)
+    got = E.eval_ops(kind, param, torch.zeros((1, 2), dtype=torch.float64, device="cuda"),
+                     torch.ones(1, dtype=torch.float64, device="cuda"), pts, 1 << R.VAL | 1 << R.DX).cpu().numpy()
+    one = E.eval_rows(kind, param, torch.zeros((1, 2), dtype=torch.float64, device="cuda"),
+                      torch.ones(1, dtype=torch.float64, device="cuda"), pts, R.DX)[0].cpu().numpy()
+    fin = r[:-4].astype(np.longdouble)
+    lg = np.log(fin) if kind == R.THIN_PLATE else np.longdouble(1)
+    val = fin ** np.longdouble(m) * lg
+    der = fin ** np.longdouble(m - 1) * (2 * param * lg + 1 if kind == R.THIN_PLATE else m)
+    size = fin ** np.longdouble(m - 1) * (2 * param * np.abs(lg) + 1 if kind == R.THIN_PLATE else m)
+    # a rounding or two of the power (pow: within 1 ulp), one of each product,
+    # within an ulp of log and one of the sum: 4 ulps
+    eps = np.finfo(float).eps
+    assert (np.abs(got[R.VAL][:-4] - val) <= 4 * eps * np.abs(val)).all()
+    for d in (got[R.DX], one):
+        assert (np.abs(d[:-4] - der) <= 4 * eps * size).all()
+        assert d[-4] == 0.0 and d[-3] == np.inf and np.isnan(d[-1])
+    assert got[R.VAL][-4] == 0.0 and got[R.VAL][-3] == np.inf and got[R.VAL][-2] == 0.0 and np.isnan(got[R.VAL][-1])
+
+
 @pytest.mark.parametrize("kind,param", C.KINDS)
 @pytest.mark.parametrize("N,P", [(5, 1), (2049, 5), (33, 2047), (40, 2049)])
 def test_gradient_in_one_evaluation(kind, param, N, P):
