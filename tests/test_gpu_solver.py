@@ -198,6 +198,31 @@ def test_radial_powers(kind, param):
     assert got[R.VAL][-4] == 0.0 and got[R.VAL][-3] == np.inf and got[R.VAL][-2] == 0.0 and np.isnan(got[R.VAL][-1])
 
 
+@pytest.mark.parametrize("eps", [1e-70, 1e-3, 0.7, 4.0, 1e5, 1e40])
+def test_multiquadric_derivatives(eps):
+    """Value, gradient and Laplacian of the multiquadric at one centre, at
+    ordinary distances (one reciprocal for both quotients) and at extreme ones
+    (divisions), against extended precision."""
+    from updes_amd import engine as E
+    rng = np.random.default_rng(7)
+    r = 2.0 ** np.concatenate([rng.uniform(-4, 4, 500), rng.uniform(-250, 120, 300),
+                               np.linspace(-1, 1, 50) - np.log2(eps), np.linspace(99, 101, 50) - np.log2(eps)])
+    r = r[(r < 1e150) & (eps * r < 1e45)]
+    pts = torch.zeros((r.size, 2), dtype=torch.float64, device="cuda")
+    pts[:, 0] = torch.as_tensor(r)
+    z, one = torch.zeros((1, 2), dtype=torch.float64, device="cuda"), torch.ones(1, dtype=torch.float64, device="cuda")
+    got = [E.eval_rows(R.MULTIQUADRIC, eps, z, one, pts, t)[0].cpu().numpy() for t in (R.VAL, R.DX, R.LAP)]
+    X, e2 = r.astype(np.longdouble), np.longdouble(eps * eps)
+    s = np.sqrt(1 + e2 * X * X)
+    f1, g2 = e2 / s, -(e2 * X / s) ** 2 / s
+    mach = np.finfo(float).eps
+    # 1 + e2 r^2 to an ulp, its root, the quotients (s^3 costs four more), a product
+    assert (np.abs(got[0] - s) <= 2 * mach * s).all()
+    assert (np.abs(got[1] - f1 * X) <= 4 * mach * f1 * X).all()
+    tiny = np.finfo(float).tiny  # (e2^2 r^2 may leave the normal range beside f1)
+    assert (np.abs(got[2] - (g2 + 2 * f1)) <= 8 * mach * (np.abs(g2) + 2 * f1) + tiny).all()
+
+
 @pytest.mark.parametrize("kind,param", C.KINDS)
 @pytest.mark.parametrize("N,P", [(5, 1), (2049, 5), (33, 2047), (40, 2049)])
 def test_gradient_in_one_evaluation(kind, param, N, P):
