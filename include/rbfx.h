@@ -242,7 +242,7 @@ int rbfx_getrs_status(int64_t n, void* d_work, size_t work_bytes, void* stream);
  * reference: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * n is at most RBFX_GETRS_NOALLOC_MAX_N (larger n: RBFX_ERR_ARG, nothing
- * queued); the array (about 2 MB) is held on every device the call runs on
+ * queued); the array (4.8 MB) is held on every device the call runs on
  * until the process ends.  All calls on one device share it: calls that
  * overlap on one GPU race.  A device-side wait that expired leaves NaN in
  * d_b (there is no status query for this variant).                        */
@@ -392,9 +392,8 @@ int rbfx_set_panel_groups(int max_groups);
 
 /* ---- tuning / test hook -----------------------------------------------------
  * Panels of rbfx_getrf_* with at least `rows` rows use 16-wide leaves instead
- * of 64-wide ones (process-wide; 0 = the default: 28,000 rows for FP64, none
- * for FP32; a negative value disables them).  No counterpart in the
- * reference.                                                               */
+ * of 64-wide ones (process-wide; 0 = the default: none; a negative value
+ * disables them).  No counterpart in the reference.                        */
 int rbfx_set_narrow_leaf_rows(int64_t rows);
 
 /* ---- test hook --------------------------------------------------------------

@@ -725,9 +725,9 @@ __device__ inline bool ld_row_entry(const unsigned long long* row, int c, unsign
 // record), the owner sends the reciprocal pivot along, one wave does the
 // polling, the reduction takes 32-bit DPP steps, and the interchanges are
 // replayed in registers.  One 64-wide leaf, averaged over the leaves of an
-// LU, FP64 / FP32: 248 / 217 us at n = 10,000 (375 / 349 us with the row
+// LU, FP64 / FP32: 234 / 209 us at n = 10,000 (375 / 349 us with the row
 // stored and waited for first, every thread polling, 64-bit DPP steps and
-// the replay in LDS); FP32 at n = 40,000, beside the trailing update: 431 us
+// the replay in LDS); FP32 at n = 40,000, beside the trailing update: 453 us
 // (643 us).
 template <typename T, int ROWS, int W, int NT>
 __global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {

@@ -105,10 +105,10 @@ __device__ inline void pin_kind(Kern& k) {
 
 // r^(m - DROP).  Whole exponents at ordinary distances are products carried
 // with their rounding errors, so the result is rounded once (largest error
-// 1.00 x 2^-53 for r^4 to r^16, pow 1.98); other exponents, and distances whose power could leave the range of
-// normal numbers, take pow.  One gradient component at 40,007 points of 10,000
-// centres: 0.69 ms for r^5 and 1.10 ms for r^11, 2.6 ms with pow; K of 12,106
-// unknowns for r^5 0.66 ms, 1.41 ms with pow.
+// 1.00 x 2^-53 for r^4 to r^16, pow 1.98); other exponents, and distances whose
+// power could leave the range of normal numbers, take pow.  One gradient
+// component at 40,007 points of 10,000 centres: 0.69 ms for r^5 and 1.10 ms for
+// r^11, 2.6 ms with pow; K of 12,106 unknowns for r^5 0.66 ms, 1.41 ms with pow.
 template <int DROP>
 __device__ inline double radial_power(const Kern& k, double r) {
   if (k.im != 0 && r >= 0x1p-60 && r <= 0x1p60) {
