@@ -43,6 +43,24 @@ def test_gemv_matches_numpy(trans, m, n, lda, alpha, beta):
     assert np.abs(got - ref).max() <= 1e-14 * scale * max(1, (m if trans else n) ** 0.5)
 
 
+@pytest.mark.parametrize("n", [1, 255, 257, 2048, 2049, 4095, 4096, 8192, 8193, 20001])
+@pytest.mark.parametrize("m,beta", [(1, 0.0), (3, -0.5), (2047, 1.0)])
+def test_gemv_few_long_rows(m, n, beta):
+    """Product with a workgroup per row (256 threads, 1,024 from 4,096 columns,
+    batches of eight and their remainders) against NumPy in FP64."""
+    L = _lib()
+    rng = np.random.default_rng(m + 3 * n)
+    A, x, y0 = rng.standard_normal((m, n)), rng.standard_normal(n), rng.standard_normal(m)
+    dA, dx = torch.as_tensor(A).cuda(), torch.as_tensor(x).cuda()
+    dy = torch.as_tensor(y0 if beta else np.full(m, np.nan)).cuda()
+    L.check(L.lib().rbfx_gemv_f64(0, m, n, 2.0, L.ptr(dA), n, L.ptr(dx), beta, L.ptr(dy), None, 0, L.stream()))
+    ref = 2.0 * (A @ x) + (beta * y0 if beta else 0.0)
+    # at most n / 256 + 16 sums in sequence on the device, NumPy's pairwise or
+    # blocked ones no more than that: each within eps / 2 of the terms' magnitudes
+    bound = (n / 256 + 32) * np.finfo(float).eps * (2.0 * np.abs(A) @ np.abs(x) + np.abs(beta * y0))
+    assert (np.abs(dy.cpu().numpy() - ref) <= bound).all()
+
+
 @pytest.mark.parametrize("m", [1, 3, 4, 31, 32, 33, 63, 64, 65])
 @pytest.mark.parametrize("n,lda,beta", [(1, 1, 0.0), (63, 64, 1.0), (65, 65, 0.0), (4097, 4100, -0.5)])
 def test_gemv_transposed_few_rows(m, n, lda, beta):

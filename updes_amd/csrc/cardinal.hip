@@ -776,10 +776,11 @@ __global__ void card_reduce_final_kernel(int64_t M, int64_t nblocks, const doubl
                                          const double* __restrict__ G, double* __restrict__ out) {
   __shared__ double sums[kCardMaxM];
   const int t = threadIdx.x;
-  if (t < M) {
+  for (int m = 0; m < M; ++m) {  // (one wave, a lane per partial)
     double s = 0.0;
-    for (int64_t b = 0; b < nblocks; ++b) s += part[b * M + t];
-    sums[t] = s;
+    for (int64_t b = t; b < nblocks; b += 64) s += part[b * M + m];
+    s = wave_sum(s);
+    if (t == 0) sums[m] = s;
   }
   __syncthreads();
   if (t < M) {
