@@ -479,3 +479,70 @@ def test_expired_sweep_wait_fails_fast_and_the_next_solve_recovers():
     res = aa @ x - b.cpu().numpy()
     assert np.isfinite(x).all()
     assert np.abs(res).max() < 1e-3 * np.linalg.norm(aa, 1) * np.linalg.norm(x, 1) * n / 100
+
+
+def _guarded_getrf(a, dtype, wait=None):
+    """info, pivots and whether the memory around the matrix is untouched, of
+    a factorisation inside a larger allocation, with garbage in the workspace
+    and in the pivots before the call."""
+    from updes_amd import engine as E
+    L = _lib()
+    n = a.shape[0]
+    ld = E._ld(n)
+    pad = 640 * ld                        # more rows than a panel's interchanges could reach
+    flat = torch.full((pad + n * ld + pad,), 12345.0, dtype=dtype, device="cuda")
+    m = flat[pad:pad + n * ld].view(n, ld)
+    m[:, :n] = torch.as_tensor(a).to(dtype).cuda()
+    ipiv = torch.full((n,), 1 << 40, dtype=torch.int64, device="cuda")
+    info = torch.full((1,), 77, dtype=torch.int32, device="cuda")
+    nbytes = 8 if dtype == torch.float64 else 4
+    ws = L.workspace(L.lib().rbfx_getrf_workspace(n, nbytes), "cuda").fill_(0x7f)
+    fn = L.lib().rbfx_getrf_f64 if nbytes == 8 else L.lib().rbfx_getrf_f32
+    if wait is not None:
+        L.check(L.lib().rbfx_set_wait_seconds(wait))
+    try:
+        L.check(fn(n, L.ptr(m), ld, L.ptr(ipiv), L.ptr(ws), ws.numel(), L.ptr(info), L.stream()))
+        torch.cuda.synchronize()
+    finally:
+        if wait is not None:
+            L.check(L.lib().rbfx_set_wait_seconds(-1.0))
+    around = bool((flat[:pad] == 12345.0).all()) and bool((flat[pad + n * ld:] == 12345.0).all())
+    return int(info.item()), ipiv.cpu().numpy(), around
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [65, 300, 603, 1100, 4200])
+@pytest.mark.parametrize("where", ["row", "first column", "late column"])
+def test_getrf_of_a_non_finite_matrix_stays_inside_it(dtype, n, where):
+    """A leaf without a finite candidate stops early: the factorisation reports
+    info = -1 (RbfxError in Python), its interchanges stay inside the matrix
+    (memory around it unchanged) and the pivots are well formed.  A NaN row
+    loses every pivot until the last column; one panel and several, recursive
+    and leaf-by-leaf panels, leaves of one workgroup and of many."""
+    from updes_amd import engine as E
+    L = _lib()
+    a = _random_well(n, 3 * n)
+    if where == "row":
+        a[n // 3] = np.nan
+    else:
+        a[:, 0 if where == "first column" else n - n // 4] = np.nan
+    info, ipiv, around = _guarded_getrf(a, dtype)
+    assert info == -1
+    assert around
+    assert (ipiv >= np.arange(n)).all() and (ipiv < n).all()
+    m = torch.zeros((n, E._ld(n)), dtype=dtype)
+    m[:, :n] = torch.as_tensor(a).to(dtype)
+    with pytest.raises(L.RbfxError):
+        E.LU(m.cuda(), n)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_getrf_whose_waits_expire_stays_inside_the_matrix(dtype):
+    """With a wait bound of 0 a leaf of several workgroups gives up wherever a
+    record is not there at once: every kernel still ends, the memory around the matrix
+    is unchanged, and info and the pivots are well formed."""
+    n = 2100
+    info, ipiv, around = _guarded_getrf(_random_well(n, 1), dtype, wait=0.0)
+    assert info in (0, -1)
+    assert around
+    assert (ipiv >= np.arange(n)).all() and (ipiv < n).all()

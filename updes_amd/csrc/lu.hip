@@ -827,6 +827,21 @@ __global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {
       }
     }
   };
+  // A leaf that stops early (a NaN column, an expired wait) moves no row: the
+  // launches after it, already queued, index rows with its moves and pivots,
+  // so workgroup 0 leaves well-formed ones on every way out.
+  auto stop = [&]() {
+    if (g != 0) return;
+    if (tid < w) {
+      a.ipiv[tid] = a.r0 + tid;
+      a.moves[tid] = tid;
+      a.moves[kPanelWMax + tid] = tid;
+    }
+    if (tid == 0) {
+      a.moves[2 * kPanelWMax] = a.o;
+      a.moves[2 * kPanelWMax + 1] = w;
+    }
+  };
   // the rows have arrived: without this the loop would wait for every memory
   // operation in flight at its top, the published row's stores included
   __builtin_amdgcn_s_waitcnt(0xF70);
@@ -924,7 +939,10 @@ __global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {
     const T* urow = &s_row[0][0] + (G > 1 ? kRowLds : 0) + kOff;
     const unsigned long long k2 = G > 1 ? s_k2 : k1;
     const T piv = urow[0], rpiv = urow[W];
-    if (k2 == kKeyBad) return;
+    if (k2 == kKeyBad) {
+      stop();
+      return;
+    }
     if (k2 == 0) {
       // no finite candidate anywhere (NaN column): every workgroup sees the
       // same key, so all of them leave here together
@@ -932,6 +950,7 @@ __global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {
         *a.info = -1;
         __hip_atomic_store(a.status, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
+      stop();
       return;
     }
     const int wq = G > 1 ? kKeyMaxGroups - 1 - (int)((k2 >> 11) & (kKeyMaxGroups - 1)) : 0;
@@ -939,6 +958,7 @@ __global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {
     if (wq >= G || wi >= (int)a.m) {
       // a key that names no row cannot come from the records: stop
       if (tid == 0) __hip_atomic_store(a.status, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      stop();
       return;
     }
     if (tid == 0) {
@@ -1201,7 +1221,9 @@ __global__ __launch_bounds__(256) void panel_apply_kernel(T* __restrict__ A, int
 // first rows, relative to the leaf's first row, its column and width).  Each
 // leaf's moves are one parallel step: content[t] is the row now at position
 // t < W, and positions past the panel sit in a hash table once a winner came
-// from there.  (Replaying the 512 interchanges one by one took 50-150 us.)
+// from there.  At most W positions are ever in the table, so a probe ends well
+// before kPlanSlots steps; the loop is bounded all the same.  (Replaying the
+// 512 interchanges one by one took 50-150 us.)
 constexpr int kSwapMax = 512;
 constexpr int kPlanSlots = 2048;
 
@@ -1224,7 +1246,7 @@ __global__ __launch_bounds__(256) void panel_finish_kernel(InvArgs<T> v, const i
   __syncthreads();
   auto slot_of = [&](int p, bool insert) -> int {
     unsigned h = ((unsigned)p * 2654435761u) >> 21;
-    for (;; h = (h + 1) & (kPlanSlots - 1)) {
+    for (int probe = 0; probe < kPlanSlots; ++probe, h = (h + 1) & (kPlanSlots - 1)) {
       const int k = key[h];
       if (k == p) return (int)h;
       if (insert && k == -1) {
@@ -1236,13 +1258,15 @@ __global__ __launch_bounds__(256) void panel_finish_kernel(InvArgs<T> v, const i
         if (old == p) return (int)h;
       }
     }
+    return -1;
   };
   for (int l = 0; l < nl; ++l, moves += kMoveStride) {
     const int o = moves[2 * kPanelWMax], w = moves[2 * kPanelWMax + 1];
     int top = 0, low = 0, to = -1;
     if (tid < w) {
       const int p = o + moves[tid];
-      top = p < W ? content[p] : held[slot_of(p, true)];
+      const int at = p < W ? -1 : slot_of(p, true);
+      top = p < W ? content[p] : at < 0 ? p : held[at];
       to = o + moves[kPanelWMax + tid];
       low = content[o + tid];
     }
@@ -1251,10 +1275,11 @@ __global__ __launch_bounds__(256) void panel_finish_kernel(InvArgs<T> v, const i
       content[o + tid] = top;
       // a displaced row goes where a winner from below the leaf came from
       if (to >= o + w) {
+        const int at = to < W ? -1 : slot_of(to, false);
         if (to < W)
           content[to] = low;
-        else
-          held[slot_of(to, false)] = low;
+        else if (at >= 0)
+          held[at] = low;
       }
     }
     __syncthreads();
