@@ -16,6 +16,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "sweep_order.h"
 
 namespace rbfx {
 
@@ -333,10 +334,11 @@ __global__ void sbcond_kernel(int64_t nblk, const double* __restrict__ part, dou
 
 // ctl[0] ticket, ctl[1] superblocks solved, ctl[2] status of the solve; the
 // s-th processed superblock counts its solved chunks in word 3 of the
-// 128-byte line ctl[kCtlLine (s + 1) ..].  Superblocks complete in order (each
-// folds its predecessor), so ctl[1] >= k means superblocks 0 .. k-1 are solved:
-// what workgroups whose turn is far off poll (one thread each); the next
-// superblock's workgroups poll their predecessor's solution itself.
+// 128-byte line ctl[kCtlLine (s + 1) ..].  Superblocks are counted in order
+// (count_solved), so ctl[1] >= k means that the plain solution of superblocks
+// 0 .. k-1 has arrived: what workgroups whose turn is far off poll (one thread
+// each); the next superblock's workgroups poll their predecessor's solution
+// itself.
 // tags: four arrays of n published values (2n words each): solution,
 // accumulated values, and for refined blocks first solution and residual.
 //
@@ -761,13 +763,18 @@ publish:
     publish(0, oI + rc0 + tid, x);
     st_coh(y + oI + rc0 + tid, x);
   }
+  // (read while the stores drain: usually the predecessor is counted by now)
+  const unsigned before = tid == 0 ? ld_coh(solved) : 0u;
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if (tid == 0) {
-    // the superblock's last chunk to finish counts it solved
-    if (__hip_atomic_fetch_add(parts + 3, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)NCH - 1)
-      __hip_atomic_fetch_add(solved, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if (tid == 0)
+    count_solved(
+        (unsigned)s, (unsigned)NCH,
+        [&]() { return __hip_atomic_fetch_add(parts + 3, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); },
+        [&](unsigned want) {
+          return before >= want || wait_for([&]() { return ld_coh(solved) >= want; }, false);
+        },
+        [&](unsigned v) { st_coh(solved, v); });
 }
 
 // Clears the ticket, the superblocks' control lines and the tags of the four
