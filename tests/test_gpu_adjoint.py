@@ -183,3 +183,27 @@ def test_checkpointed_bptt_matches_full_graph():
     gmax = b.grad.abs().max().item()
     print("fd check: |fd - g| / max|g| = %.3e (max|g| %.3e)" % (abs(fd - b.grad[k].item()) / gmax, gmax))
     assert abs(fd - b.grad[k].item()) <= 1e-6 * gmax
+
+
+@pytest.mark.parametrize("P", [1, 5])
+def test_field_results_can_be_changed_in_place(P):
+    """Values, gradients and Laplacians of a field that needs gradients take
+    changes in place (they are no views), and backpropagate through them."""
+    import updes_amd as u
+    rng = np.random.default_rng(P)
+    ctr = torch.as_tensor(rng.uniform(0, 1, (7, 2))).cuda()
+    pts = torch.as_tensor(rng.uniform(0, 1, (P, 2))).cuda()
+    c0 = torch.as_tensor(rng.standard_normal(10)).cuda()
+    for fn in (u.value_vec, u.gradient_vec, u.laplacian_vec):
+        grads = []
+        for inplace in (False, True):
+            c = c0.clone().requires_grad_(True)
+            v = fn(pts, c, ctr, u.polyharmonic)
+            if inplace:
+                v.mul_(3.0)
+                v[0] = 0.0
+            else:
+                v = torch.cat([torch.zeros_like(v[:1]), 3.0 * v[1:]])
+            v.sum().backward()
+            grads.append(c.grad)
+        assert torch.equal(grads[0], grads[1])

@@ -71,7 +71,7 @@ class EvalOp(torch.autograd.Function):
     @staticmethod
     def forward(ctx, coeffs, kind, param, centers, points, op):
         ctx.save = (kind, param, centers, points, op, coeffs.numel() - centers.shape[0])
-        return E.eval_rows(kind, param, centers, coeffs, points, op)[0]
+        return E.eval_op(kind, param, centers, coeffs, points, op)
 
     @staticmethod
     def backward(ctx, g):
@@ -86,7 +86,8 @@ class EvalGrad(torch.autograd.Function):
     @staticmethod
     def forward(ctx, coeffs, kind, param, centers, points):
         ctx.save = (kind, param, centers, points, coeffs.numel() - centers.shape[0])
-        return E.eval_rows(kind, param, centers, coeffs, points, L.DX, 2).t().contiguous()
+        # (a tensor of its own: autograd refuses changes in place of a result that is a view)
+        return E.eval_rows(kind, param, centers, coeffs, points, L.DX, 2).t().clone(memory_format=torch.contiguous_format)
 
     @staticmethod
     def backward(ctx, g):

@@ -263,6 +263,12 @@ def eval_ops(kind, param, centers, coeffs, points, mask):
     return _eval_into(kind, param, centers, coeffs, points, mask, out, 0)
 
 
+def eval_op(kind, param, centers, coeffs, points, op):
+    """(P,) values of one operator alone."""
+    out = torch.empty(points.numel() // 2, dtype=torch.float64, device=centers.device)
+    return _eval_into(kind, param, centers, coeffs, points, 1 << op, out, op)
+
+
 def eval_rows(kind, param, centers, coeffs, points, op, count=1):
     """(count, P) values of the operators op .. op + count - 1 alone."""
     out = torch.empty((count, points.numel() // 2), dtype=torch.float64, device=centers.device)
