@@ -546,3 +546,48 @@ def test_getrf_whose_waits_expire_stays_inside_the_matrix(dtype):
     assert info in (0, -1)
     assert around
     assert (ipiv >= np.arange(n)).all() and (ipiv < n).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("groups", [0, 6])
+def test_getrf_panel_solves_round_once(dtype, groups):
+    """The inverse X of a panel's unit-lower block L11 and the solves with its
+    64 x 64 diagonal blocks are formed in FP64 and rounded once.  L11 itself
+    stands in the matrix (unit diagonal, smaller entries below: no row moves
+    and the elimination is exact), beside identity columns, where U then shows
+    X (a product with the identity is exact) or, inside the panel, the solve."""
+    from updes_amd import engine as E
+    L = _lib()
+    n, half = 1100, 2.0 ** (-53 if dtype == torch.float64 else -24)
+    rng = np.random.default_rng(5)
+    low = np.tril(rng.uniform(-0.25, 0.25, (512, 512)).astype(np.float32).astype(np.float64), -1) + np.eye(512)
+    for inside in (False, True):
+        a = np.eye(n)
+        if inside:
+            a[:64, :64] = low[:64, :64]
+            a[:64, 64:128] = np.eye(64)
+        else:
+            a[:512, :512] = low
+            a[:512, 512:1024] = np.eye(512)
+        m = torch.zeros((n, E._ld(n)), dtype=dtype)
+        m[:, :n] = torch.as_tensor(a).to(dtype)
+        L.check(L.lib().rbfx_set_panel_groups(groups))
+        try:
+            lu = E.LU(m.cuda(), n)
+        finally:
+            L.check(L.lib().rbfx_set_panel_groups(0))
+        assert np.array_equal(lu.ipiv.cpu().numpy(), np.arange(n))
+        got = lu.a[:, :n].double().cpu().numpy()
+        T = low[:64, :64] if inside else low
+        w = len(T)
+        assert np.array_equal(np.tril(got[:w, :w], -1) + np.eye(w), T)
+        got = got[:w, 64:128] if inside else got[:w, 512:1024]
+        X = sla.solve_triangular(T, np.eye(w), lower=True, unit_diagonal=True)
+        # FP64 arithmetic: at most 512 terms per entry, forward error through |X| |L| |X|
+        noise = 512 * 2.0 ** -53 * (np.abs(X) @ np.abs(T) @ np.abs(X))
+        bound = half * np.abs(X) + noise
+        for b in range(0, w, 64):          # rows below use the rounded rows above
+            r = slice(b, b + 64)
+            D = sla.solve_triangular(T[r, r], np.eye(64), lower=True, unit_diagonal=True)
+            bound[r, :b] += np.abs(D) @ (np.abs(T[r, :b]) @ bound[:b, :b])
+        assert (np.abs(got - X) <= bound).all(), (inside, np.max(np.abs(got - X) / np.maximum(bound, 1e-300)))

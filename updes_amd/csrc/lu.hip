@@ -616,9 +616,12 @@ __device__ inline void tri_inv16(F&& L, double (*out)[17]) {
 // layout) <- inv(L) acc for the 64 x 64 unit-lower L, given its entries below
 // the 16 x 16 diagonal blocks and those blocks' inverses.  An accumulator
 // tile is the B operand of the next product as it stands: MFMA k-step s takes
-// row Mma<T>::row(lane, s), element s of the tile.
-template <typename T, typename F>
-__device__ inline void tri_solve64(typename Mma<T>::acc_t (&acc)[4], F&& L, const double (*inv)[16][17]) {
+// row row(lane, s), element s of the tile.  In FP64 for factors of either
+// type, so that a solve or an inverse of FP32 factors is rounded once, at its
+// end.
+typedef Mma<double> MmaTri;
+template <typename F>
+__device__ inline void tri_solve64(MmaTri::acc_t (&acc)[4], F&& L, const double (*inv)[16][17]) {
   const int lane = threadIdx.x & 63, m = lane & 15;
 #pragma unroll
   for (int I = 0; I < 4; ++I) {
@@ -626,10 +629,10 @@ __device__ inline void tri_solve64(typename Mma<T>::acc_t (&acc)[4], F&& L, cons
     for (int J = 0; J < I; ++J)
 #pragma unroll
       for (int s = 0; s < 4; ++s)
-        acc[I] = Mma<T>::mma(-L(16 * I + m, 16 * J + Mma<T>::row(lane, s)), acc[J][s], acc[I]);
-    typename Mma<T>::acc_t u = {};
+        acc[I] = MmaTri::mma(-(double)L(16 * I + m, 16 * J + MmaTri::row(lane, s)), acc[J][s], acc[I]);
+    MmaTri::acc_t u = {};
 #pragma unroll
-    for (int s = 0; s < 4; ++s) u = Mma<T>::mma((T)inv[I][m][Mma<T>::row(lane, s)], acc[I][s], u);
+    for (int s = 0; s < 4; ++s) u = MmaTri::mma(inv[I][m][MmaTri::row(lane, s)], acc[I][s], u);
     acc[I] = u;
   }
 }
@@ -649,12 +652,12 @@ __device__ inline void inverse_rows(const InvArgs<T>& v, int q, double (*inv)[16
       },
       inv[wv]);
   __syncthreads();
-  typename Mma<T>::acc_t acc[4];
+  MmaTri::acc_t acc[4];
 #pragma unroll
   for (int I = 0; I < 4; ++I)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      acc[I][e] = q == v.b && 16 * I + Mma<T>::row(lane, e) == 16 * wv + m ? T(1) : T(0);
+      acc[I][e] = q == v.b && 16 * I + MmaTri::row(lane, e) == 16 * wv + m ? 1.0 : 0.0;
   const int c0 = kTri * q + 16 * wv + m;  // this lane's column of X
   for (int k = q; k < v.b; ++k) {
 #pragma unroll
@@ -662,6 +665,7 @@ __device__ inline void inverse_rows(const InvArgs<T>& v, int q, double (*inv)[16
       T bv[4], av[4][4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
+        // (any order of k serves both operands: FP32 entries in runs of four)
         const int kk = kTri * k + 16 * kb + Mma<T>::row(lane, s);
         bv[s] = v.X[(int64_t)kk * v.ldx + c0];
 #pragma unroll
@@ -670,17 +674,17 @@ __device__ inline void inverse_rows(const InvArgs<T>& v, int q, double (*inv)[16
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int I = 0; I < 4; ++I) acc[I] = Mma<T>::mma(-av[I][s], bv[s], acc[I]);
+        for (int I = 0; I < 4; ++I) acc[I] = MmaTri::mma(-(double)av[I][s], (double)bv[s], acc[I]);
     }
   }
-  tri_solve64<T>(
+  tri_solve64(
       acc, [&](int i, int k) -> T { return i < v.w ? D[(int64_t)i * v.lda + k] : T(0); }, inv);
 #pragma unroll
   for (int I = 0; I < 4; ++I)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int r = 16 * I + Mma<T>::row(lane, e);
-      if (r < v.w && (q < v.b || 16 * wv + m < v.w)) v.X[(int64_t)(kTri * v.b + r) * v.ldx + c0] = acc[I][e];
+      const int r = 16 * I + MmaTri::row(lane, e);
+      if (r < v.w && (q < v.b || 16 * wv + m < v.w)) v.X[(int64_t)(kTri * v.b + r) * v.ldx + c0] = (T)acc[I][e];
     }
 }
 
@@ -1196,20 +1200,20 @@ __global__ __launch_bounds__(256) void panel_apply_kernel(T* __restrict__ A, int
   tri_inv16([&](int i, int k) -> double { return (double)Ls[16 * wv + i][16 * wv + k]; }, inv[wv]);
   __syncthreads();
   const int m = lane & 15;
-  typename Mma<T>::acc_t acc[4];
+  MmaTri::acc_t acc[4];
 #pragma unroll
   for (int I = 0; I < 4; ++I)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc[I][e] = Ss[16 * I + Mma<T>::row(lane, e)][16 * wv + m];
-  tri_solve64<T>(
+    for (int e = 0; e < 4; ++e) acc[I][e] = Ss[16 * I + MmaTri::row(lane, e)][16 * wv + m];
+  tri_solve64(
       acc, [&](int i, int k) -> T { return Ls[i][k]; }, inv);
   if (16 * wv + m >= nc) return;
 #pragma unroll
   for (int I = 0; I < 4; ++I)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int r = 16 * I + Mma<T>::row(lane, e);
-      if (r < w) C[(int64_t)r * lda + 16 * wv + m] = acc[I][e];
+      const int r = 16 * I + MmaTri::row(lane, e);
+      if (r < w) C[(int64_t)r * lda + 16 * wv + m] = (T)acc[I][e];
     }
 }
 
