@@ -477,3 +477,20 @@ def test_rhs_abi_matches_oracle(fs):
     got = assemble_q(rhs, bcs, uc, u.polyharmonic, M, None).cpu().numpy()
     ref = OA.assemble_q(oc, xi[:, 0] * xi[:, 1] + 1.0, arrs)
     assert np.abs(got - ref).max() <= 1e-14 * np.abs(ref).max()
+
+
+def test_multiquadric_whose_square_of_eps_squared_overflows():
+    """eps^4 past the range of FP64: value and gradient stay right, and the
+    second derivative's term overflows to -inf as in the closed form."""
+    from updes_amd import engine as E
+    eps = 2.0 ** 260
+    r = 2.0 ** np.array([-200.0, -255.0, -262.0])
+    pts = torch.zeros((3, 2), dtype=torch.float64, device="cuda")
+    pts[:, 0] = torch.as_tensor(r)
+    z, one = torch.zeros((1, 2), dtype=torch.float64, device="cuda"), torch.ones(1, dtype=torch.float64, device="cuda")
+    got = [E.eval_op(R.MULTIQUADRIC, eps, z, one, pts, t).cpu().numpy() for t in (R.VAL, R.DX, R.LAP)]
+    with np.errstate(invalid="ignore"):
+        ref = R.rbf_ops(R.MULTIQUADRIC, eps, r[:, None], 0.0 * r[:, None], np.zeros((1, 1)), np.zeros((1, 1)))[..., 0]
+    for t, op in enumerate((R.VAL, R.DX)):
+        assert (np.abs(got[t] - ref[op]) <= 8 * np.finfo(float).eps * np.abs(ref[op])).all()
+    assert (ref[R.LAP] == -np.inf).all() and (got[2] == -np.inf).all()

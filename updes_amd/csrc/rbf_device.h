@@ -27,6 +27,7 @@ struct Kern {
   double e2;   // eps^2
   double phi0; // value at r = 0
   bool fast;   // a == 1 closed forms without pow
+  bool mid;    // multiquadric: e2 leaves room for quot_mid (e2^2 in range)
 };
 
 constexpr int kMaxPower = 16;
@@ -48,6 +49,7 @@ __host__ __device__ inline Kern make_kern(int kind, double param) {
   } else {
     k.phi0 = 1.0;  // gaussian, multiquadric, inverse multiquadric
   }
+  k.mid = k.e2 >= 0x1p-200 && k.e2 <= 0x1p500;
   k.im = k.m >= 3.0 && k.m <= kMaxPower && k.m == (int)k.m ? (int)k.m : 0;
   return k;
 }
@@ -158,7 +160,7 @@ __device__ inline double quot_mid(double a, double s, double y) {
 // 0.51 ms with the library's root and two divisions.
 __device__ inline void multiquadric(const Kern& k, double r, double& phi, double& f1, double& g2) {
   const double x = __builtin_fma(k.e2 * r, r, 1.0), num = -k.e2 * k.e2 * r * r;
-  if (x <= 0x1p200 && k.e2 >= 0x1p-200 && num <= -0x1p-400) {
+  if (k.mid && x <= 0x1p200 && num <= -0x1p-400) {
     const double s = sqrt_mid(x), y = recip_mid(s);
     phi = s;
     f1 = quot_mid(k.e2, s, y);
