@@ -591,3 +591,21 @@ def test_getrf_panel_solves_round_once(dtype, groups):
             D = sla.solve_triangular(T[r, r], np.eye(64), lower=True, unit_diagonal=True)
             bound[r, :b] += np.abs(D) @ (np.abs(T[r, :b]) @ bound[:b, :b])
         assert (np.abs(got - X) <= bound).all(), (inside, np.max(np.abs(got - X) / np.maximum(bound, 1e-300)))
+
+
+@pytest.mark.parametrize("m", [1, 5, 64])
+@pytest.mark.parametrize("n", [131071, 131072, 131073, 300001])
+def test_gemv_transposed_few_long_rows(m, n):
+    """Transposed product of few rows on both sides of 131,072 columns (one
+    kernel; chunks and their sum) against NumPy in FP64."""
+    L = _lib()
+    rng = np.random.default_rng(m + n)
+    A, x, y0 = rng.standard_normal((m, n)), rng.standard_normal(m), rng.standard_normal(n)
+    dA, dx, dy = (torch.as_tensor(v).cuda() for v in (A, x, y0))
+    ws = L.workspace(L.lib().rbfx_gemv_workspace(1, m, n), "cuda")
+    L.check(L.lib().rbfx_gemv_f64(1, m, n, -1.0, L.ptr(dA), n, L.ptr(dx), 0.5, L.ptr(dy), L.ptr(ws), ws.numel(),
+                                  L.stream()))
+    ref = -(A.T @ x) + 0.5 * y0
+    # m products and m + 1 sums, each within eps / 2 of the terms' magnitudes, on both sides
+    bound = (m + 2) * np.finfo(float).eps * (np.abs(A).T @ np.abs(x) + np.abs(0.5 * y0))
+    assert (np.abs(dy.cpu().numpy() - ref) <= bound).all()

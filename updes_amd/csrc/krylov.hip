@@ -186,13 +186,16 @@ __global__ void gemv_t_finish_kernel(int64_t n, int64_t chunks, const double* __
 }
 
 // The same for at most kGvFewRows rows (combinations of the basis vectors of
-// GMRES), whole: a workgroup takes 64 columns, wave w their rows w, w + 4, ...
+// GMRES) of at most kGvFewCols columns, whole: a workgroup takes 64 columns, wave w their rows w, w + 4, ...
 // with eight loads in flight a thread, and writes y itself.  Bound by latency:
 // inside GMRES 4 us for 2 to 4 rows of 10,006 columns, the chunks above and their
 // finish 40 us; back to back on resident rows 8.4 to 9.5 us against 11.1 to 11.8 at
 // every number of rows from 1 to 64 and 600 to 40,006 columns (two launches
-// against one), past which the chunks share the work.
-constexpr int64_t kGvFewRows = 64;
+// against one), past which the chunks share the work.  Columns past kGvFewCols
+// are bound by bandwidth, where the chunks' 16-byte loads are ahead: 5 rows of
+// 100,000 columns 10.7 against 13.0 us, of 150,000 both 13.1, of 1,000,000 38
+// against 23.
+constexpr int64_t kGvFewRows = 64, kGvFewCols = 1 << 17;
 __global__ __launch_bounds__(kGvThreads) void gemv_t_few_kernel(int64_t m, int64_t n, double alpha,
                                                                 const double* __restrict__ A, int64_t lda,
                                                                 const double* __restrict__ x, double beta,
@@ -275,7 +278,7 @@ int gemv_launch(int trans, int64_t m, int64_t n, double alpha, const double* A, 
     return RBFX_OK;
   }
   RBFX_REQUIRE(part != nullptr, "gemv^T needs a workspace");
-  if (m <= kGvFewRows) {
+  if (m <= kGvFewRows && n <= kGvFewCols) {
     hipLaunchKernelGGL(gemv_t_few_kernel, dim3((unsigned)ceil_div(n, 64)), dim3(kGvThreads), 0, s, m, n, alpha, A,
                        lda, x, beta, y);
     RBFX_CHECK_LAUNCH();
