@@ -1415,21 +1415,13 @@ constexpr int kPanelMaxRows = 3;  // rows per thread of the register-resident le
 // 2.52 / 2.62 ms; FP32 n = 450 1.29 / 1.39 ms, n = 1024 3.10 / 3.49 ms.
 template <typename T>
 static bool lone_leaf(int64_t m, int w, int& nt, LeafShape& shape) {
-  static const struct { int nt, rows; } f64[] = {{kPanelThreads, 1}, {512, 1}, {768, 1}};
-  static const struct { int nt, rows; } f32[] = {{kPanelThreads, 1}, {512, 1}, {1024, 1}};
-  auto pick = [&](const auto& table) {
-    for (const auto& e : table)
-      if (m <= (int64_t)e.nt * e.rows) {
-        nt = e.nt;
-        shape.rows = e.rows;
-        shape.G = 1;
-        shape.R = m;
-        return true;
-      }
-    return false;
-  };
-  if (w <= kPanelWNarrow && m > kPanelThreads) return false;
-  return sizeof(T) == 8 ? pick(f64) : pick(f32);
+  constexpr int widest = sizeof(T) == 8 ? 768 : 1024;
+  if (m > (w <= kPanelWNarrow ? kPanelThreads : widest)) return false;
+  nt = m <= kPanelThreads ? kPanelThreads : m <= 512 ? 512 : widest;
+  shape.rows = 1;
+  shape.G = 1;
+  shape.R = m;
+  return true;
 }
 
 template <typename T>
@@ -1545,7 +1537,7 @@ constexpr int64_t kStageAlign = 16;
 // and columns [col, col+ncols): staged copy of A12, then one GEMM.
 template <typename T>
 static int trsm(LuCtx<T>& c, int64_t r0, int W, const T* X, int64_t ldx, int64_t col, int64_t ncols, T* tmp,
-                int64_t tmp_elems, bool on_panel_stream = false) {
+                int64_t tmp_elems) {
   if (ncols <= 0) return RBFX_OK;
   int st;
   const int pid = prof_start(sizeof(T) == 8 ? "trsm_f64" : "trsm_f32", c.s);
@@ -1557,8 +1549,7 @@ static int trsm(LuCtx<T>& c, int64_t r0, int W, const T* X, int64_t ldx, int64_t
     hipLaunchKernelGGL((copy_block_kernel<T>), dim3((unsigned)std::min<int64_t>(ceil_div(w, 256), 64), W),
                        dim3(256), 0, c.s, B + off, c.lda, W, w, tmp, ldt);
     RBFX_CHECK_LAUNCH();
-    if ((st = gemm_launch<T, 1>(W, w, W, T(1), X, ldx, tmp, ldt, T(0), B + off, c.lda, c.s,
-                                on_panel_stream && sizeof(T) == 4, !c.recursive)))
+    if ((st = gemm_launch<T, 1>(W, w, W, T(1), X, ldx, tmp, ldt, T(0), B + off, c.lda, c.s, false, !c.recursive)))
       return st;
   }
   prof_stop(pid, c.s, 2.0 * W * W * ncols, 3.0 * sizeof(T) * W * ncols);
@@ -1583,10 +1574,12 @@ static int panel(LuCtx<T>& c, int64_t r0, int W, T* X, int64_t ldx, LuScratch<T>
   inv.X = X;
   inv.ldx = ldx;
   int nl = (W + c.wleaf - 1) / c.wleaf;
-  if (c.recursive) {
-    c.nleaves = 0;
-    if ((st = panel_recursive(c, r0, W, r0, W, X, ldx))) return st;
-    nl = c.nleaves;
+  if constexpr (sizeof(T) == 8) {
+    if (c.recursive) {
+      c.nleaves = 0;
+      if ((st = panel_recursive(c, r0, W, r0, W, X, ldx))) return st;
+      nl = c.nleaves;
+    }
   }
   for (int o = 0, l = 0; !c.recursive && o < W; o += c.wleaf, ++l) {
     const int w = std::min(c.wleaf, W - o);
@@ -1648,7 +1641,7 @@ static int panel_recursive(LuCtx<T>& c, int64_t pc0, int pw, int64_t r0, int W, 
     if ((st = leaf(c, r0, o, W, moves, v))) return st;
     v.X = X;
     v.ldx = ldx;
-    const int pid = prof_start(sizeof(T) == 8 ? "panel_apply_f64" : "panel_apply_f32", c.s);
+    const int pid = prof_start("panel_apply_f64", c.s);
     hipLaunchKernelGGL((panel_apply_kernel<T, false>),
                        dim3((unsigned)(ceil_div(o, kTri) + ceil_div(pw - o - W, kTri) + 1)), dim3(256), 0, c.s,
                        c.A + r0 * c.lda + pc0, c.lda, o, W, pw, (const int*)moves, v);
@@ -1659,7 +1652,7 @@ static int panel_recursive(LuCtx<T>& c, int64_t pc0, int pw, int64_t r0, int W, 
   const int W1 = std::max(8, (W / 2 + 7) / 8 * 8);
   const int W2 = W - W1;
   if ((st = panel_recursive(c, pc0, pw, r0, W1, X, ldx))) return st;
-  if ((st = trsm(c, r0, W1, X, ldx, r0 + W1, W2, c.panel_tmp, (int64_t)kNB * kNB, true))) return st;
+  if ((st = trsm(c, r0, W1, X, ldx, r0 + W1, W2, c.panel_tmp, (int64_t)kNB * kNB))) return st;
   const int64_t m2 = c.n - r0 - W1;
   const T* L21 = c.A + (r0 + W1) * c.lda + r0;
   if ((st = gemm<T>(m2, W2, W1, T(-1), L21, c.lda, c.A + r0 * c.lda + r0 + W1, c.lda, T(1),
@@ -1669,7 +1662,7 @@ static int panel_recursive(LuCtx<T>& c, int64_t pc0, int pw, int64_t r0, int W, 
   if ((st = panel_recursive(c, pc0, pw, r0 + W1, W2, X22, ldx))) return st;
   // L21 (rows r0+W1 .. r0+W) is final now: later pivots only move rows
   // >= r0+W
-  const int pid = prof_start(sizeof(T) == 8 ? "trtri_f64" : "trtri_f32", c.s);
+  const int pid = prof_start("trtri_f64", c.s);
   if ((st = gemm_launch<T, 2>(W2, W1, W1, T(1), L21, c.lda, X, ldx, T(0), c.panel_tmp, W1, c.s, true, false)))
     return st;
   st = gemm_launch<T, 2>(W2, W1, W2, T(-1), X22, ldx, c.panel_tmp, W1, T(0), X + (int64_t)W1 * ldx, ldx, c.s, true,

@@ -751,8 +751,7 @@ __global__ __launch_bounds__(kSweepThreads) void sbsweep_kernel(const TF* __rest
     __syncthreads();
     reduce_rows(pr);
     __syncthreads();
-    // L_KK has a unit diagonal that is not stored: its x0 term
-    const T r_r = tid < nr ? xs[rc0 + tid] - row_value(tid) - (WHICH == 0 ? xs2[rc0 + tid] : T(0)) : T(0);
+    const T r_r = tid < nr ? xs[rc0 + tid] - row_value(tid) : T(0);
     if (!exchange(3, r_r, xs2, [&]() { load_D(dv); })) return;
     apply(dv, xs2);
     __syncthreads();
