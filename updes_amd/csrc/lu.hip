@@ -646,11 +646,15 @@ __device__ inline void inverse_rows(const InvArgs<T>& v, int q, double (*inv)[16
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, m = lane & 15;
   const T* Lb = v.P + (int64_t)kTri * v.b * v.lda;  // rows of the block
   const T* D = Lb + kTri * v.b;
-  tri_inv16(
-      [&](int i, int k) -> double {
-        return 16 * wv + i < v.w ? (double)D[(int64_t)(16 * wv + i) * v.lda + 16 * wv + k] : 0.0;
-      },
-      inv[wv]);
+  // rows past the block read its last one and count as zero (in the diagonal
+  // block columns past it read its first): loads inside the matrix without a
+  // branch, which the compiler issues together
+  auto entry = [&](const T* rows, int i, int k) -> T {
+    const T x = rows[(int64_t)(i < v.w ? i : v.w - 1) * v.lda + k];
+    return i < v.w ? x : T(0);
+  };
+  auto diag = [&](int i, int k) -> T { return entry(D, i, k < v.w ? k : 0); };
+  tri_inv16([&](int i, int k) -> double { return (double)diag(16 * wv + i, 16 * wv + k); }, inv[wv]);
   __syncthreads();
   MmaTri::acc_t acc[4];
 #pragma unroll
@@ -669,7 +673,7 @@ __device__ inline void inverse_rows(const InvArgs<T>& v, int q, double (*inv)[16
         const int kk = kTri * k + 16 * kb + Mma<T>::row(lane, s);
         bv[s] = v.X[(int64_t)kk * v.ldx + c0];
 #pragma unroll
-        for (int I = 0; I < 4; ++I) av[I][s] = 16 * I + m < v.w ? Lb[(int64_t)(16 * I + m) * v.lda + kk] : T(0);
+        for (int I = 0; I < 4; ++I) av[I][s] = entry(Lb, 16 * I + m, kk);
       }
 #pragma unroll
       for (int s = 0; s < 4; ++s)
@@ -677,8 +681,7 @@ __device__ inline void inverse_rows(const InvArgs<T>& v, int q, double (*inv)[16
         for (int I = 0; I < 4; ++I) acc[I] = MmaTri::mma(-(double)av[I][s], (double)bv[s], acc[I]);
     }
   }
-  tri_solve64(
-      acc, [&](int i, int k) -> T { return i < v.w ? D[(int64_t)i * v.lda + k] : T(0); }, inv);
+  tri_solve64(acc, diag, inv);
 #pragma unroll
   for (int I = 0; I < 4; ++I)
 #pragma unroll
