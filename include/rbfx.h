@@ -372,7 +372,11 @@ int rbfx_profile_end(rbfx_prof_entry* out, int max_entries, int* n_entries);
 
 /* ---- test hook --------------------------------------------------------------
  * C = beta C + alpha A B (row-major, beta 0 or 1) with the MFMA kernel that
- * performs the LU trailing updates.                                         */
+ * performs the LU trailing updates.  Where the leading dimensions and the
+ * addresses are multiples of 16 bytes and ldb, ldc >= n rounded up to 16
+ * bytes, B and C are read in 16-byte units: the last row up to the end of the
+ * unit that holds its last column, whose other entries may hold anything and
+ * are not written.                                                          */
 int rbfx_gemm_f64(int64_t m, int64_t n, int64_t k, double alpha, const double* d_A,
                   int64_t lda, const double* d_B, int64_t ldb, double beta, double* d_C,
                   int64_t ldc, void* stream);

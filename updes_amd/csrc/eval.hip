@@ -321,9 +321,9 @@ __global__ __launch_bounds__(kEvThreads) void eval_t_kernel(Kern k, int64_t N, i
 
 // The same for at most kChunkPoints points, each centre's sum in a fixed
 // order: four quarters of the points, each summed in sequence, added in
-// order.  The adjoint of implicit time stepping calls it at these sizes, where
-// kappa ~ 1e10 turns another order of summation into 2e-9 of its gradients
-// (60 x 60 nodes, 8 steps).  A workgroup takes kChunkCentres centres: all its
+// order.  The limit keeps results: the adjoint of implicit time stepping calls
+// it at these sizes, where kappa ~ 1e10 turns another order of summation, no
+// less accurate, into 2e-9 of its gradients (60 x 60 nodes, 8 steps).  A workgroup takes kChunkCentres centres: all its
 // threads form the pairs of a tile (kChunkTile points of every quarter) in
 // LDS while its first wave adds the tile before, a lane per (centre, quarter).
 // 88 us for 3,480 points and 3,600 centres (r^3, value); 285 us when each lane

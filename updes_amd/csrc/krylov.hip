@@ -29,8 +29,9 @@ constexpr int kRateWindow = 24;
 // y[i] = alpha * sum_j A[i][j] x[j] + beta * y[i]: one block of NT threads per
 // row, with eight pairs of loads in flight a thread.  Few long rows are bound
 // by the latency of a row in one workgroup and take 1024 threads: 1 to 32 rows
-// of 40,006 columns 11 us, 20 us with 256 threads (10,006 columns, back to back, 7.7
-// and 8.0).  More rows than CUs fill the chip with 256 (2,000 rows of 4,096
+// of 40,006 columns 11 us, 20 us with 256 threads, alone on the GPU (10,006 columns,
+// back to back, 7.7 and 8.0); inside GMRES at 40,006 columns 13.7 us, 53 us
+// with 256 threads and one load in flight each.  More rows than CUs fill the chip with 256 (2,000 rows of 4,096
 // columns 11.3 us, 12.7 us with 1024).
 constexpr int64_t kGvLongRow = 4096;
 template <int NT>

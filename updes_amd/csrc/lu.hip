@@ -7,13 +7,18 @@
 // once: P K = L U.
 //
 // Structure per outer panel of NB columns (k0 .. k0+NB):
-//   1. recursive panel factorisation: halves down to 64-wide leaves; each
-//      leaf runs as ONE launch of co-resident workgroups that keep their rows
-//      of the leaf in registers and agree on every pivot through one exchange per
-//      column (every workgroup publishes its best row and a tagged record,
-//      all of them poll the records and pick the same winner);
-//      the leaves apply their interchanges to the panel's other columns and
-//      invert their diagonal blocks; the splits join those inverses;
+//   1. panel factorisation, leaf by leaf (64 columns): a leaf runs as ONE
+//      launch of co-resident workgroups that keep their rows of the leaf in
+//      registers and agree on every pivot through one exchange per column
+//      (every workgroup publishes its best row and a tagged record, all of
+//      them poll the records and pick the same winner); a second launch
+//      applies its interchanges to the panel's other columns and solves for
+//      U12 of its rows, and one product updates what is right and below.  The
+//      inverse of the panel's unit-lower block grows by a row block per leaf,
+//      beside the next one; its last block and the plan of the panel's
+//      interchanges are one launch.  (FP64 systems of up to kRecursiveRows
+//      rows: by recursive halving, whose splits solve and join inverses with
+//      products.)
 //   2. row interchanges of the columns outside the panel through a
 //      gather/scatter plan (row-major rows are contiguous, so a swap is a
 //      coalesced copy);
@@ -494,10 +499,11 @@ constexpr int kRowWords = sizeof(T) / 4;
 template <typename T>
 constexpr int kRowStride = (kPanelWMax + 2) * kRowWords<T>;
 // Narrow leaves, on request only (rbfx_set_narrow_leaf_rows): a 16-wide FP64
-// leaf (72 VGPRs) shares a CU with two trailing-update workgroups (2 x 216
-// VGPRs per SIMD), a 64-wide one (202) displaces one of them.  That paid when
-// a panel cost more than the update beside it; now an FP64 LU takes 832 ms with
-// them and 835 ms without at n = 40,006, 466 and 464 ms at n = 32,006.
+// leaf (72 VGPRs) displaces less of the trailing update than a 64-wide one
+// (246).  It paid when a panel cost more than the update beside it and two
+// update workgroups left it room (2 x 216 of 512, now 2 x 224); now an FP64 LU
+// takes 832 ms with them and 835 ms without at n = 40,006, 466 and 464 ms at
+// n = 32,006.
 constexpr int kPanelWNarrow = 16;
 static std::atomic<int64_t> g_narrow_leaf_rows{0};
 // A pivot record (two 64-bit words) owns a 128-byte line: every workgroup
@@ -732,10 +738,14 @@ __device__ inline bool ld_row_entry(const unsigned long long* row, int c, unsign
 // record), the owner sends the reciprocal pivot along, one wave does the
 // polling, the reduction takes 32-bit DPP steps, and the interchanges are
 // replayed in registers.  One 64-wide leaf, averaged over the leaves of an
-// LU, FP64 / FP32: 234 / 209 us at n = 10,000 (375 / 349 us with the row
+// LU, FP64 / FP32: 233 / 198 us at n = 10,000 (375 / 349 us with the row
 // stored and waited for first, every thread polling, 64-bit DPP steps and
-// the replay in LDS); FP32 at n = 40,000, beside the trailing update: 453 us
-// (643 us).
+// the replay in LDS); FP32 at n = 40,000, beside the trailing update: 420 us
+// (643 us).  The workgroups that form rows of the inverse cost registers:
+// FP64 246 VGPRs with one row per thread (170 without), FP32 178 / 234 / 288
+// with one / two / three rows (98 / 194 / 260), so an FP32 leaf of two or
+// three rows per thread displaces one of the two update workgroups (2 x 152 of
+// 512) on its CU.
 template <typename T, int ROWS, int W, int NT>
 __global__ __launch_bounds__(NT) void panel_kernel(PanelArgs<T> a) {
   static_assert(W <= kPanelWMax && W <= 64, "leaf wider than the candidate rows");
@@ -1621,12 +1631,15 @@ static int panel(LuCtx<T>& c, int64_t r0, int W, T* X, int64_t ldx, LuScratch<T>
 
 // FP64 systems of at most this many rows take the recursive panels: U12 by
 // the inverse of the half panel's whole diagonal block, as opposed to block
-// substitution.  Both are backward stable (same ||P A - L U||), but implicit
-// time stepping at these sizes goes through tens of solves with kappa(K) ~
-// 1e10, where another rounding of the factors moves its results by up to 2e-9
-// (60 x 60 nodes, 8 steps); larger systems and the FP32 factors (which only
-// precondition) take the leaf-by-leaf panels, which are faster: FP64 LU at
-// n = 10,006 47.0 against 60.1 ms.
+// substitution.  The limit keeps results, it buys neither speed nor accuracy:
+// both forms are backward stable (same ||P A - L U||), and on 16 time
+// steppings of 66 x 66 to 90 x 90 nodes neither is nearer to the 64-bit
+// solution (median error of the gradients 2.0e-9 with either); but with kappa(K) ~
+// 1e10 through tens of solves another rounding of the factors moves the
+// results by up to 2e-9, and systems of this size keep theirs.  It costs 16.9
+// against 15.4 ms at 4,096 and 4,097 unknowns; larger systems and the FP32
+// factors (which only precondition) take the leaf-by-leaf panels: FP64 LU at
+// n = 10,006 46.4 against 60.1 ms.
 constexpr int64_t kRecursiveRows = 4096;
 constexpr int kMaxLeaves = kNB / 8;  // the recursion splits no narrower than 8
 

@@ -3,12 +3,13 @@
 //
 // Replaces the solve phase of lineax QR (updes/operators.py:612-613) and the
 // inv(A) @ v products (updes/assembly.py:410,430).  Blocked, synchronisation-
-// free sweep: one workgroup per 64-row block row, taken in dependency order
-// from an atomic ticket; each workgroup folds in the off-diagonal tiles of the
-// blocks already solved (a monotone completion counter tells it how far it
-// may go), then applies the precomputed inverse of its diagonal block and
-// publishes its slice.  Row-major storage makes the no-transpose tiles
-// row-contiguous and the transposed tiles column-coalesced.
+// free sweep: superblocks of 512 rows, 16 workgroups of 32 rows each, taken in
+// dependency order from an atomic ticket; each workgroup folds in the
+// off-diagonal tiles of the superblocks already solved, exchanges its
+// accumulated values with the superblock's other workgroups, applies its rows
+// of the precomputed inverse of the diagonal superblock and publishes its
+// slice.  Row-major storage makes the no-transpose tiles row-contiguous and
+// the transposed tiles column-coalesced.
 #include <algorithm>
 #include <climits>
 #include <vector>
@@ -110,14 +111,15 @@ __global__ void scatter_perm_kernel(const double* __restrict__ y, const int64_t*
 
 // ---- superblock sweep ---------------------------------------------------------
 // The chain of a blocked triangular solve is what bounds it at these sizes:
-// every exchange between workgroups is a coherent store, a counter and a
-// poll through the memory side of the chip (~2 us each).  The superblock
+// every exchange between workgroups is a coherent store and a poll through the
+// memory side of the chip (~1.2 us each).  The superblock
 // sweep makes the chain n/SB steps instead of n/TB: the solution advances by
 // SB = 512 rows at a time, each superblock's rows solved with its 512 x 512
 // diagonal inverse (built once per factorisation by sbinv_kernel), by NCH
 // workgroups of CH rows:
-//   1. fold the tiles of the superblocks already solved, in solve order
-//      (each superblock counts its solved chunks), into private partial sums;
+//   1. fold the tiles of the superblocks already solved, in solve order, into
+//      private partial sums (the predecessor's solution from its published
+//      values, earlier ones once the count of solved superblocks covers them);
 //   2. publish the chunk's CH accumulated values b - sum;
 //   3. once all NCH chunks of the superblock are in, apply rows of its
 //      diagonal inverse to the superblock's SB values and publish the CH
