@@ -609,3 +609,23 @@ def test_gemv_transposed_few_long_rows(m, n):
     # m products and m + 1 sums, each within eps / 2 of the terms' magnitudes, on both sides
     bound = (m + 2) * np.finfo(float).eps * (np.abs(A).T @ np.abs(x) + np.abs(0.5 * y0))
     assert (np.abs(dy.cpu().numpy() - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("at,value", [(0, -1), (99, 98), (299, 300)])
+def test_getrs_prepare_refuses_pivots_before_any_work(dtype, at, value):
+    """An invalid pivot is refused with nothing queued: the inverses' buffer
+    and the permutation stay as they were."""
+    from updes_amd import engine as E
+    L = _lib()
+    n = 300
+    m = torch.eye(n, E._ld(n), dtype=dtype, device="cuda")
+    ipiv = torch.arange(n, device="cuda")
+    ipiv[at] = value
+    perm = torch.full((n,), -7, dtype=torch.int64, device="cuda")
+    dinv = torch.full((L.lib().rbfx_getrs_dinv_elems(n),), 3.5, dtype=torch.float64, device="cuda")
+    fn = L.lib().rbfx_getrs_prepare_f64 if dtype == torch.float64 else L.lib().rbfx_getrs_prepare_f32
+    st = fn(n, L.ptr(m), E._ld(n), L.ptr(ipiv), L.ptr(perm), L.ptr(dinv), None, 0, L.stream())
+    assert st != 0 and b"invalid pivot" in L.lib().rbfx_last_error()
+    torch.cuda.synchronize()
+    assert bool((dinv == 3.5).all()) and bool((perm == -7).all())

@@ -982,6 +982,9 @@ static int prepare(int64_t n, const T* LU, int64_t lda, const int64_t* ipiv, int
   std::vector<int64_t> hp(n), pm(n);
   RBFX_HIP(hipMemcpyAsync(hp.data(), ipiv, n * sizeof(int64_t), hipMemcpyDeviceToHost, s));
   RBFX_HIP(hipStreamSynchronize(s));
+  // (checked before anything is queued)
+  for (int64_t i = 0; i < n; ++i)
+    RBFX_REQUIRE(hp[i] >= i && hp[i] < n, "invalid pivot ipiv[%lld] = %lld", (long long)i, (long long)hp[i]);
   // the inverses run while the host replays the interchanges
   const int64_t nsb = ceil_div(n, (int64_t)SB);
   double* d512 = dinv + dinv64_elems(n);
@@ -999,11 +1002,7 @@ static int prepare(int64_t n, const T* LU, int64_t lda, const int64_t* ipiv, int
                      (const double*)part, cond);
   RBFX_CHECK_LAUNCH();
   for (int64_t i = 0; i < n; ++i) pm[i] = i;
-  for (int64_t i = 0; i < n; ++i) {
-    const int64_t p = hp[i];
-    RBFX_REQUIRE(p >= i && p < n, "invalid pivot ipiv[%lld] = %lld", (long long)i, (long long)p);
-    std::swap(pm[i], pm[p]);
-  }
+  for (int64_t i = 0; i < n; ++i) std::swap(pm[i], pm[hp[i]]);
   RBFX_HIP(hipMemcpyAsync(perm, pm.data(), n * sizeof(int64_t), hipMemcpyHostToDevice, s));
   RBFX_HIP(hipStreamSynchronize(s));  // pm must outlive the copy
   return RBFX_OK;
